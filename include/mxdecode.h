@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define MX_ABI_VERSION 18
+#define MX_ABI_VERSION 19
 
 typedef enum mx_status {
     MX_OK = 0,
@@ -256,6 +256,22 @@ int mx_paged_attn_decode_noalloc(const uint16_t* q, int64_t q_sb, int64_t q_sh, 
                                  int32_t D, int32_t block_size, int32_t num_pool_blocks, float scale, uint16_t* out,
                                  int64_t o_sb, int64_t o_sh, int32_t chunk_tokens, uint32_t flags, int32_t* err,
                                  void* stream);
+
+/* Causal attention of a prompt over contiguous K and V, with the weights:
+ * weights[b, h, i, j] = softmax_j(scale * q[b, h, i] . k[b, h / G, j]) over
+ * j <= i + S - P, rounded to the element type (0 at the masked j), and
+ * out[b, i, h] = sum_j weights[b, h, i, j] v[b, h / G, j] of the rounded
+ * weights, fp32 accumulation. Replaces the eager branch of
+ * block_paged_attention_forward (runtime/phase2/block_paged_attention.py:50-60)
+ * for a prompt: one launch, nothing else written.
+ * q: fp16 (bf16 with MX_PA_BF16) [B, Hq, P, D] with strides (q_sb, q_sh, q_st, 1);
+ * k, v: [B, Hkv, S, D] with their strides; out: [B, P, Hq, D] contiguous;
+ * weights: [B, Hq, P, S] contiguous; S >= P, D in {64, 128}, Hq = G * Hkv.
+ * Pointers 16-byte aligned, strides non-negative multiples of 8; scale > 0. */
+int mx_prefill_attn(const uint16_t* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const uint16_t* k, int64_t k_sb,
+                    int64_t k_sh, int64_t k_st, const uint16_t* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int32_t B,
+                    int32_t Hq, int32_t Hkv, int32_t P, int32_t S, int32_t D, float scale, uint16_t* out,
+                    uint16_t* weights, uint32_t flags, void* stream);
 
 /* Calibration probe (no reference counterpart; used by bench.py): the K/V reads
  * of mx_paged_attn_decode over the same block tables and lengths, without the

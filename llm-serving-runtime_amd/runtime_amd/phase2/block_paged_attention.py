@@ -5,7 +5,8 @@ registered as ``ALL_ATTENTION_FUNCTIONS["block_paged"]`` with
 ``config._attn_implementation = "block_paged"`` (``runtime/phase2/worker_server.py:274-281``).
 When decode metadata is set, ``q_len == 1`` and the query is on a device, the
 fused HIP kernel runs and ``[B, 1, Hq, D]`` is returned (``:37-48``); otherwise
-eager attention on the gathered K/V (prefill, ``:50-60``).
+attention on the gathered K/V (prefill, ``:50-60``): one HIP launch for a causal prompt
+on the device (``_prefill_kernel_takes``), else the eager chain.
 
 Difference kept on purpose: transformers 5.x hands a custom attention
 implementation that has no registered mask function ``attention_mask=None``
@@ -20,7 +21,12 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from .paged_attention_hip import get_paged_decode_batch_metadata, paged_attention_decode_batched
+from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode
+from torch.utils._python_dispatch import _get_current_dispatch_mode
+
+from . import _hip
+from .paged_attention_hip import _DTYPE_FLAGS, get_paged_decode_batch_metadata, paged_attention_decode_batched
 
 
 def repeat_kv(hidden_states: torch.Tensor, n_rep: int) -> torch.Tensor:
@@ -37,6 +43,59 @@ def _causal_block(q_len: int, kv_len: int, device: torch.device) -> torch.Tensor
     return torch.arange(kv_len, device=device).view(1, -1) > qpos
 
 
+def _rows_aligned(t: torch.Tensor) -> bool:
+    """Whether the prefill kernel can read ``t [B, H, T, D]`` with 16-byte loads."""
+    return (t.stride(3) == 1 and t.data_ptr() % 16 == 0
+            and all(t.stride(i) % 8 == 0 for i in range(3) if t.shape[i] > 1))
+
+
+def _prefill_kernel_takes(query, key, value, scaling, num_kv_groups) -> bool:
+    """Whether ``mx_prefill_attn`` gives this call's causal attention. It takes plain device tensors
+    outside autograd, tracing, function transforms and autocast (the eager chain is what those
+    see), of one 16-bit dtype and a supported head_dim, with at least as many keys as queries (a
+    query before the first key has no visible token: the eager chain's softmax over nothing) and a
+    positive scale (the kernel masks scaled scores with -inf)."""
+    if not all(type(t) is torch.Tensor and t.is_cuda and t.dim() == 4 for t in (query, key, value)):
+        return False
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_autocast_enabled("cuda"):
+        return False
+    if (_get_current_dispatch_mode() is not None or _get_current_function_mode() is not None
+            or forward_ad._current_level >= 0):
+        return False
+    if any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in (query, key, value)):
+        return False
+    if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad):
+        return False
+    b, hq, q_len, d = query.shape
+    _, hkv, kv_len, _ = key.shape
+    return (query.dtype in _DTYPE_FLAGS and key.dtype == query.dtype and value.dtype == query.dtype
+            and query.device == key.device == value.device
+            and value.shape == key.shape and key.shape[0] == b and key.shape[3] == d and d in (64, 128)
+            and hkv > 0 and hq == hkv * num_kv_groups and b > 0 and 2 <= q_len <= kv_len
+            and isinstance(scaling, (int, float)) and 0.0 < scaling < 3e38
+            and b * hq * q_len < 1 << 30 and kv_len < 1 << 30
+            and kv_len * max(key.stride(2), value.stride(2)) < 1 << 31
+            and _rows_aligned(query) and _rows_aligned(key) and _rows_aligned(value))
+
+
+def _prefill(query, key, value, scaling) -> tuple[torch.Tensor, torch.Tensor]:
+    """Causal attention of a prompt: ``out [B, P, Hq, D]`` and the weights ``[B, Hq, P, S]``."""
+    b, hq, q_len, d = query.shape
+    hkv, kv_len = key.shape[1], key.shape[2]
+    out = torch.empty((b, q_len, hq, d), dtype=query.dtype, device=query.device)
+    weights = torch.empty((b, hq, q_len, kv_len), dtype=query.dtype, device=query.device)
+
+    def strides(t):  # the stride of a dimension of one is never used and may be anything
+        return [t.stride(i) if t.shape[i] > 1 else 0 for i in range(3)]
+
+    with torch.cuda.device(query.device):
+        _hip.check(_hip.load().mx_prefill_attn(
+            query.data_ptr(), *strides(query), key.data_ptr(), *strides(key), value.data_ptr(), *strides(value), b, hq,
+            hkv, q_len, kv_len, d, float(scaling), out.data_ptr(), weights.data_ptr(), _DTYPE_FLAGS[query.dtype],
+            _hip.stream_handle(query.device)), "mx_prefill_attn")
+    return out, weights
+
+
 def block_paged_attention_forward(module, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                                   attention_mask: torch.Tensor | None, scaling: float, dropout: float = 0.0, **kwargs):
     num_kv_groups = getattr(module, "num_key_value_groups", 1)
@@ -45,6 +104,10 @@ def block_paged_attention_forward(module, query: torch.Tensor, key: torch.Tensor
         attn_output = paged_attention_decode_batched(query=query, metadata=meta, num_kv_groups=num_kv_groups,
                                                      scaling=scaling)
         return attn_output.transpose(1, 2).contiguous(), None
+
+    if (attention_mask is None and not (dropout > 0.0 and module.training)
+            and _prefill_kernel_takes(query, key, value, scaling, num_kv_groups)):
+        return _prefill(query, key, value, scaling)
 
     key_states = repeat_kv(key, num_kv_groups)
     value_states = repeat_kv(value, num_kv_groups)
