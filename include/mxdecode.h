@@ -409,6 +409,18 @@ int mx_kv_append(const uint16_t* k_new, const uint16_t* v_new, int64_t new_sb, i
                  int64_t kv_shead, int32_t block_size, int32_t num_pool_blocks, int32_t* err, uint8_t* used_blocks,
                  void* stream);
 
+/* The first S tokens of B rows of the pool, contiguous: k_out and v_out
+ * [B, Hkv, S, D] (16-bit elements) from per-layer views of the layout
+ * mx_kv_append writes. seq_lens (int32 [B], nullable: S for every row): tokens
+ * past a row's length are zero. A token whose block is outside the table or the
+ * pool is zero and sets bit 0 of the nullable err word. Replaces
+ * GpuKVBlockPool.gather_layer / gather_layer_batch
+ * (runtime/phase2/paged_kv_kernel.py:252-309). */
+int mx_kv_gather(const uint16_t* k_pool, const uint16_t* v_pool, int64_t kv_sblk, int64_t kv_shead,
+                 const int32_t* block_tables, int64_t bt_sb, int32_t max_blocks, const int32_t* seq_lens, int32_t B,
+                 int32_t S, int32_t Hkv, int32_t D, int32_t block_size, int32_t num_pool_blocks, uint16_t* k_out,
+                 uint16_t* v_out, int32_t* err, void* stream);
+
 /* From one fused QKV projection row per sequence (fp16 [B, (Hq + 2*Hkv) * D],
  * row stride qkv_stride; heads in the order q, k, v): rotate q and k with
  * rotate-half RoPE at position positions[b] (pairs i, i + D/2 use

@@ -72,6 +72,10 @@ SIGNATURES = {
         [_p, _p, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i64, _i32, _i32, _p,
          _p, _p],
     ),
+    "mx_kv_gather": (
+        ctypes.c_int,
+        [_p, _p, _i64, _i64, _p, _i64, _i32, _p, _i32, _i32, _i32, _i32, _i32, _i32, _p, _p, _p, _p],
+    ),
     "mx_qkv_rope_append": (
         ctypes.c_int,
         [_p, _i64, _i32, _i32, _i32, _i32, _p, _i32, _p, _p, _i64, _p, _p, _i64, _i64, _p, _i64, _i32, _i32, _i32,

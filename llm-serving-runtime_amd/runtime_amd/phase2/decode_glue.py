@@ -3,6 +3,8 @@
 * :func:`kv_append` — scatter new K/V states into a layer of a
   :class:`GpuKVBlockPool` (``GpuKVBlockPool.write_tokens_batch`` semantics,
   ``runtime/phase2/paged_kv_kernel.py:176-227``) in one launch;
+* :func:`kv_gather` — the reverse: whole rows of a layer as contiguous K and V in one launch
+  (``GpuKVBlockPool.gather_layer``, ``paged_kv_kernel.py:252-309``);
 * :func:`qkv_rope_append` — rotate q and k of a fused QKV projection output and
   append k, v at each row's position (the HF decoder layer's
   ``apply_rotary_pos_emb`` + ``BlockPagedBatchLayer.update`` write,
@@ -154,6 +156,24 @@ def kv_append(k_layer: torch.Tensor, v_layer: torch.Tensor, block_tables: torch.
         key_states.stride(2), b, t, hkv, d, tables.data_ptr(), tables.stride(0), int(tables.shape[1]),
         starts.data_ptr(), k_layer.data_ptr(), v_layer.data_ptr(), k_layer.stride(0), k_layer.stride(1), bs, nb,
         err.data_ptr() if err is not None else None, used, _hip.stream_handle(dev)), "mx_kv_append")
+
+
+def kv_gather(k_layer: torch.Tensor, v_layer: torch.Tensor, block_tables: torch.Tensor, tokens: int,
+              seq_lens: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+    """The first ``tokens`` tokens of each row of ``block_tables [B, max_blocks]`` (int32, on the pool's
+    device): K and V as contiguous ``[B, Hkv, tokens, D]``, zero past ``seq_lens[b]`` when given. Block
+    ids must be in the pool (a token of one that is not comes back zero)."""
+    dev = k_layer.device
+    nb, hkv, bs, d = k_layer.shape
+    tables = _i32(block_tables, dev)
+    b = int(tables.shape[0])
+    k, v = (torch.empty(b, hkv, tokens, d, dtype=k_layer.dtype, device=dev) for _ in range(2))
+    lens = _i32(seq_lens.reshape(-1), dev) if seq_lens is not None else None
+    _hip.check(_hip.load().mx_kv_gather(
+        k_layer.data_ptr(), v_layer.data_ptr(), k_layer.stride(0), k_layer.stride(1), tables.data_ptr(),
+        tables.stride(0), int(tables.shape[1]), lens.data_ptr() if lens is not None else None, b, tokens, hkv, d, bs, nb,
+        k.data_ptr(), v.data_ptr(), None, _hip.stream_handle(dev)), "mx_kv_gather")
+    return k, v
 
 
 def qkv_rope_append(qkv: torch.Tensor, rope: torch.Tensor, positions: torch.Tensor, q_out: torch.Tensor,

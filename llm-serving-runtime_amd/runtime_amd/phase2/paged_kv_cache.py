@@ -104,7 +104,8 @@ class BlockPagedLayer(CacheLayerMixin):
             raise IndexError(f"block table underrun: {start + kv_len} tokens in {len(self._block_ids)} blocks")
         table = self._table().view(1, -1)
         if self._seq_len_dev is None:
-            self._seq_len_dev = torch.tensor([start], dtype=torch.int32).to(self.pool.device)
+            # Filled on the device: a copy from the host would wait for the work enqueued before it.
+            self._seq_len_dev = torch.full((1,), start, dtype=torch.int32, device=self.pool.device)
         self.pool.write_tokens_batch(self.layer_idx, table, self._seq_len_dev, key_states, value_states)
         self._seq_len += kv_len
         self._seq_len_dev.add_(kv_len)
@@ -115,7 +116,23 @@ class BlockPagedLayer(CacheLayerMixin):
             return key_states, value_states
 
         set_paged_decode_batch_metadata(None)
-        return self.pool.gather_layer(self.layer_idx, self._block_ids, self._seq_len)
+        return self._rows(start, table, key_states, value_states)
+
+    def _rows(self, start: int, table: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor
+              ) -> tuple[torch.Tensor, torch.Tensor]:
+        """K and V of the row's tokens after a prefill write, ``pool.gather_layer``'s values: the new
+        states themselves when they are the whole row in the pool's dtype and every block has a place
+        of its own (nothing to read back), else gathered in one launch over the row's device table."""
+        pool = self.pool
+        if not pool._gathers_on_device() or table.dtype != torch.int32 or table.device.type != "cuda":
+            return pool.gather_layer(self.layer_idx, self._block_ids, self._seq_len)
+        ids = [int(b) for b in self._block_ids[: -(-self._seq_len // pool.block_size_tokens)]]
+        distinct = pool._touch_ids(ids)
+        if start == 0 and len(distinct) == len(ids) and all(
+                t.dtype == pool.dtype and t.device == table.device and not t.requires_grad
+                for t in (key_states, value_states)):
+            return key_states, value_states
+        return pool._gather_table(self.layer_idx, table, self._seq_len)
 
     def get_mask_sizes(self, query_length: int) -> tuple[int, int]:
         return self._seq_len + query_length, 0

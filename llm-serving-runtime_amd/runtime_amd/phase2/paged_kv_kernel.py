@@ -157,8 +157,22 @@ class GpuKVBlockPool:
         self._peak_allocated_blocks = max(self._peak_allocated_blocks, len(self._used_blocks))
 
     def _touch_blocks(self, physical_ids: torch.Tensor) -> None:
-        for physical in physical_ids.unique().tolist():
-            self._touch_block(int(physical))
+        self._touch_ids(physical_ids.unique().tolist())
+
+    def _touch_ids(self, ids: list[int]) -> set[int]:
+        """:meth:`_touch_block` of every id; the distinct ones."""
+        distinct = set(ids)
+        if distinct and (min(distinct) < 0 or max(distinct) >= self.shape.num_blocks):
+            for physical in ids:  # raises at the first id out of range
+                self._touch_block(int(physical))
+        self._used_blocks |= distinct
+        self._peak_allocated_blocks = max(self._peak_allocated_blocks, len(self._used_blocks))
+        return distinct
+
+    def _gathers_on_device(self) -> bool:
+        """Whether rows come out of the pool by ``mx_kv_gather``: 16-bit elements in 16-byte chunks."""
+        return (self.device.type == "cuda" and self.dtype in (torch.float16, torch.bfloat16)
+                and self.shape.head_dim % 8 == 0)
 
     def k_layer_view(self, layer_idx: int) -> torch.Tensor:
         """Per-layer K blocks: ``[num_blocks, num_kv_heads, block_size, head_dim]``."""
@@ -272,13 +286,22 @@ class GpuKVBlockPool:
         self._ensure_pools()
         assert self._k_pool is not None and self._v_pool is not None
         ids_list = [int(b) for b in list(block_ids)[:n_logical]]
-        for b in ids_list:
-            self._touch_block(b)
+        self._touch_ids(ids_list)
+        if self._gathers_on_device():
+            table = torch.tensor([ids_list], dtype=torch.int32).to(self.device)
+            return self._gather_table(layer_idx, table, seq_len)
         ids = torch.tensor(ids_list, device=self.device, dtype=torch.long)
         s = self.shape
         k = self._k_pool[layer_idx, ids].permute(1, 0, 2, 3).reshape(s.num_kv_heads, n_logical * bs, s.head_dim)
         v = self._v_pool[layer_idx, ids].permute(1, 0, 2, 3).reshape(s.num_kv_heads, n_logical * bs, s.head_dim)
         return k[:, :seq_len].unsqueeze(0), v[:, :seq_len].unsqueeze(0)
+
+    def _gather_table(self, layer_idx: int, table: torch.Tensor, tokens: int, seq_lens: torch.Tensor | None = None
+                      ) -> tuple[torch.Tensor, torch.Tensor]:
+        """Rows of a device table (ids checked by the caller) as ``[B, Hkv, tokens, D]``, one launch."""
+        from .decode_glue import kv_gather
+
+        return kv_gather(self.k_layer_view(layer_idx), self.v_layer_view(layer_idx), table, tokens, seq_lens)
 
     def gather_layer_batch(self, layer_idx: int, block_tables: torch.Tensor, seq_lens: torch.Tensor
                            ) -> tuple[torch.Tensor, torch.Tensor]:
@@ -288,6 +311,15 @@ class GpuKVBlockPool:
         max_seq = max(lens) if lens else 0
         if max_seq <= 0:
             raise ValueError("seq_len must be positive")
+        if self._gathers_on_device():
+            for row, n in zip(block_tables.tolist(), lens):
+                if n <= 0:
+                    raise ValueError("seq_len must be positive")
+                n_logical = math.ceil(n / self.block_size_tokens)
+                if n_logical > len(row):
+                    raise IndexError("block table underrun during gather")
+                self._touch_ids([int(i) for i in row[:n_logical]])
+            return self._gather_table(layer_idx, block_tables, max_seq, seq_lens)
         s = self.shape
         keys = torch.zeros(batch_size, s.num_kv_heads, max_seq, s.head_dim, device=self.device, dtype=self.dtype)
         values = torch.zeros_like(keys)

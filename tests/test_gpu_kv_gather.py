@@ -74,3 +74,46 @@ def test_gather_errors_follow_the_reference():
         pool.gather_layer_batch(0, torch.tensor([[1], [2]], device=DEV), torch.tensor([0, 0], device=DEV))
     with pytest.raises(IndexError):
         pool.gather_layer_batch(0, torch.tensor([[1], [2]], device=DEV), torch.tensor([16, 17], device=DEV))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("start,new,ids", [
+    (0, 1000, None), (0, 17, None), (32, 45, None), (7, 2, None),
+    (0, 40, [3, 5, 3]),  # a block listed twice: the row reads back what the later tokens wrote
+])
+def test_prefill_update_returns_the_rows_in_the_pool(dtype, start, new, ids):
+    from runtime_amd.phase2.paged_kv_cache import BlockPagedLayer
+    from runtime_amd.phase2.paged_kv_kernel import GpuKVBlockPool
+
+    hkv, bs, d = 2, 16, 64
+    pool = GpuKVBlockPool(num_blocks=80, block_size_tokens=bs, num_layers=1, num_kv_heads=hkv, head_dim=d, dtype=dtype,
+                          device=DEV)
+    gen = torch.Generator(device=DEV).manual_seed(new)
+    for view in (pool.k_layer_view(0), pool.v_layer_view(0)):
+        view.copy_(torch.randn(view.shape, generator=gen, device=DEV))
+    ids = ids or torch.randperm(80, generator=torch.Generator().manual_seed(new)).tolist()[: -(-(start + new) // bs)]
+    layer = BlockPagedLayer(pool, 0)
+    layer.set_block_ids(ids)
+    layer.set_seq_length(start)
+    k, v = (torch.randn(1, new, hkv, d, generator=gen, device=DEV).to(dtype).transpose(1, 2) for _ in range(2))
+    got = layer.update(k, v)
+    if len(set(ids)) == len(ids):
+        want = okv.gather_layer_view(pool.k_layer_view(0).cpu(), pool.v_layer_view(0).cpu(), ids, start + new)
+        assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
+        assert torch.equal(got[0][:, :, start:], k) and torch.equal(got[1][:, :, start:], v)
+    else:  # which write of a block listed twice lands last is not defined: read back, not handed through
+        want = pool.gather_layer(0, ids, start + new)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert pool.allocated_block_count() == len(set(ids))
+    assert int(layer._seq_len_dev) == start + new
+
+
+def test_prefill_update_with_a_block_outside_the_pool_raises():
+    from runtime_amd.phase2.paged_kv_cache import BlockPagedLayer
+
+    pool = _filled_pool("interleaved", 16, 2, 16, 64, 1, seed=5)
+    layer = BlockPagedLayer(pool, 0)
+    layer.set_block_ids([3, 16])
+    k = torch.randn(1, 2, 20, 64, device=DEV).half()
+    with pytest.raises(IndexError):
+        layer.update(k, k)
