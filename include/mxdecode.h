@@ -83,7 +83,7 @@ int mx_w8a16_linear(const uint16_t* x, int64_t M, int64_t K, int64_t x_stride, c
  * hand the split partials to a consumer that sums them itself (the decode
  * glue kernels below), saving mx_w8a16_linear's separate reduce launch.
  * Returns 1 for M > 128, where no partials entry exists (mx_w8a16_linear runs
- * 128-row chunks, each planned as M = 128). */
+ * one launch over all rows, its k ranges within the workspace of 128 rows). */
 int mx_w8a16_splits(int64_t M, int64_t N, int64_t K);
 
 /* The split-K part of mx_w8a16_linear without the reduction:
@@ -119,9 +119,9 @@ int mx_w8a16_linear_partials_swiglu(const uint16_t* gate_up, int64_t M, int64_t 
  * 8t + [0, 8) (scale and bias reordered the same way), quantized and packed
  * as usual. Replaces transformers' act_fn(gate_proj(x)) * up_proj(x) (reached
  * from worker_server.py:771-775) with one launch and half the output bytes.
- * Rows are processed 128 at a time: the VALU GEMV where mx_w8a16_linear would
- * take it (M <= 4 on shapes that split), else one MFMA launch that never splits
- * K, whatever mx_w8a16_splits reports for the plain projection. */
+ * The VALU GEMV where mx_w8a16_linear would take it (M <= 4 on shapes that
+ * split), else one MFMA launch that never splits K, whatever mx_w8a16_splits
+ * reports for the plain projection. */
 int mx_w8a16_gateup_swiglu(const uint16_t* x, int64_t M, int64_t K, int64_t x_stride, const uint8_t* packed,
                            const uint16_t* scale, const uint16_t* bias, uint16_t* y, int64_t I, int64_t y_stride,
                            void* stream);

@@ -22,6 +22,7 @@
 // meet in LDS. The MFMA GEMM (M > 4) splits the other way, see gemm_mfma_kernel.
 // Both apply the per-channel scale and the bias once, in the epilogue.
 #include "common.h"
+#include "w8a16_rows.h"
 #include "w8a16_tiles.h"
 
 namespace mx {
@@ -666,7 +667,7 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ p
 
 // Largest M handled by the VALU GEMV; above it the MFMA kernel runs.
 constexpr int kValuMaxM = 4;
-constexpr int kMaxRows = 128;  // rows per MFMA launch (8 m-tiles); larger M runs in chunks
+constexpr int kMaxRows = 128;  // rows per MFMA launch (8 m-tiles); more go to w8a16_rows.hip (or, past its indices, in chunks)
 // Waves per GEMV workgroup (one workgroup per n-tile, the waves taking interleaved k-tiles): 4
 // where the grid alone covers the chip (more than 256 n-tiles) or K is short or long (at most 32
 // or at least 128 k-tiles), else 8 (few workgroups that must each pull a middling K: the
@@ -763,6 +764,14 @@ constexpr int kMwMinRangeTiles = 16;
 static bool use_m_split(int MT, int NT, int KT) {
     if (!big_m_shape(NT)) return false;
     return MT >= 6 || (MT == 4 && KT / big_splits(NT, KT) >= kMwMinRangeTiles);
+}
+
+// gate||up (never split) goes to the many-row launch above 128 rows, and at 65-128 rows where the
+// M-split shape would leave more than half of the CUs without a workgroup: the Qwen2-0.5B gate||up
+// (76 workgroups) at 128 rows 13.9 -> 10.2 us on MI355X; the Llama-3-8B one (224 workgroups) takes 43
+// us here and 44-46 there.
+static bool gateup_takes_rows(int64_t M, int NT) {
+    return M > kMaxRows || (M > 64 && ceil_div(NT, kBigTiles) <= kBigGrid / 2);
 }
 
 static Plan plan_for(int M, int NT, int KT) {
@@ -1105,7 +1114,7 @@ extern "C" int mx_w8a16_pack(const int8_t* q, int64_t N, int64_t K, uint8_t* pac
 
 extern "C" size_t mx_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || N % w8a16::kTileN || K % w8a16::kTileK) return 0;
-    const int mc = (int)(M < w8a16::kMaxRows ? M : w8a16::kMaxRows);  // rows are processed in chunks
+    const int mc = (int)(M < w8a16::kMaxRows ? M : w8a16::kMaxRows);  // more rows stay within it (plan_rows)
     return w8a16::workspace_for(mc, (int)(N / w8a16::kTileN), (int)(K / w8a16::kTileK));
 }
 
@@ -1131,6 +1140,16 @@ extern "C" int mx_w8a16_linear(const uint16_t* x, int64_t M, int64_t K, int64_t 
     const int KT = (int)(K / w8a16::kTileK);
     hipStream_t st = as_stream(stream);
     float* partial = static_cast<float*>(workspace);
+    if (M > w8a16::kMaxRows && w8a16::rows_fit(M, x_stride, NT)) {
+        // Planned from the bytes the call may ask for, not from those it got: the same shape always
+        // takes the same ranges.
+        w8a16::RowsPlan rp = w8a16::plan_rows(M, NT, KT, mx_w8a16_workspace_bytes(M, N, K));
+        if (rp.KS > 1 && (!workspace || workspace_bytes < (size_t)rp.KS * M * N * sizeof(float)))
+            rp = w8a16::plan_rows(M, NT, KT, 0);
+        w8a16::launch_rows(false, rp, x, x_stride, (int)M, packed, scale, bias, y, y_stride, NT, KT, partial, st);
+        if (rp.KS > 1) w8a16::launch_reduce(partial, rp.KS, (int)M, (int)N, bias, y, y_stride, st);
+        return check_launch("mx_w8a16_linear");
+    }
     for (int64_t m0 = 0; m0 < M; m0 += w8a16::kMaxRows) {
         const int mc = (int)((M - m0) < w8a16::kMaxRows ? (M - m0) : w8a16::kMaxRows);
         const uint16_t* xc = x + m0 * x_stride;
@@ -1253,12 +1272,17 @@ extern "C" int mx_w8a16_gateup_swiglu(const uint16_t* x, int64_t M, int64_t K, i
     const int NT = (int)(2 * I / w8a16::kTileN), KT = (int)(K / w8a16::kTileK);
     if ((int64_t)NT * w8a16::kTileN != 2 * I || K * 64 > 0x7fffffff)
         return fail(MX_ERR_UNSUPPORTED, "mx_w8a16_gateup_swiglu: bad shape");
-    // Rows in chunks of at most kMaxRows, as mx_w8a16_linear: the VALU GEMV where that entry
+    // The many-row launch, or at most kMaxRows rows: the VALU GEMV where mx_w8a16_linear
     // would take it (M <= 4 on shapes that split), else one unsplit MFMA launch, also where
     // mx_w8a16_linear would split K: the epilogue needs the whole sum, and on such (small)
     // shapes one launch without K split costs less than a split launch plus a SwiGLU launch
     // (the Qwen2-0.5B MLP at batch 16).
     hipStream_t st = as_stream(stream);
+    if (w8a16::gateup_takes_rows(M, NT) && w8a16::rows_fit(M, x_stride, NT)) {
+        w8a16::launch_rows(true, w8a16::plan_rows(M, NT, KT, 0), x, x_stride, (int)M, packed, scale, bias, y, y_stride,
+                           NT, KT, nullptr, st);
+        return check_launch("mx_w8a16_gateup_swiglu");
+    }
     for (int64_t m0 = 0; m0 < M; m0 += w8a16::kMaxRows) {
         const int mc = (int)(M - m0 < w8a16::kMaxRows ? M - m0 : w8a16::kMaxRows);
         const uint16_t* xc = x + m0 * x_stride;
