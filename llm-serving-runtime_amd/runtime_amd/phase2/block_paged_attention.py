@@ -45,8 +45,10 @@ def _causal_block(q_len: int, kv_len: int, device: torch.device) -> torch.Tensor
 
 def _rows_aligned(t: torch.Tensor) -> bool:
     """Whether the prefill kernel can read ``t [B, H, T, D]`` with 16-byte loads."""
-    return (t.stride(3) == 1 and t.data_ptr() % 16 == 0
-            and all(t.stride(i) % 8 == 0 for i in range(3) if t.shape[i] > 1))
+    b, h, n, _ = t.shape
+    sb, sh, sn, unit = t.stride()
+    return (unit == 1 and t.data_ptr() % 16 == 0 and (b == 1 or sb % 8 == 0) and (h == 1 or sh % 8 == 0)
+            and (n == 1 or sn % 8 == 0))
 
 
 def _prefill_kernel_takes(query, key, value, scaling, num_kv_groups) -> bool:
@@ -55,14 +57,16 @@ def _prefill_kernel_takes(query, key, value, scaling, num_kv_groups) -> bool:
     see), of one 16-bit dtype and a supported head_dim, with at least as many keys as queries (a
     query before the first key has no visible token: the eager chain's softmax over nothing) and a
     positive scale (the kernel masks scaled scores with -inf)."""
-    if not all(type(t) is torch.Tensor and t.is_cuda and t.dim() == 4 for t in (query, key, value)):
-        return False
+    for t in (query, key, value):
+        if type(t) is not torch.Tensor or not t.is_cuda or t.dim() != 4:
+            return False
     if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_autocast_enabled("cuda"):
         return False
     if (_get_current_dispatch_mode() is not None or _get_current_function_mode() is not None
             or forward_ad._current_level >= 0):
         return False
-    if any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in (query, key, value)):
+    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+    if wrapped(query) or wrapped(key) or wrapped(value):
         return False
     if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad):
         return False
@@ -86,9 +90,10 @@ def _prefill(query, key, value, scaling) -> tuple[torch.Tensor, torch.Tensor]:
     weights = torch.empty((b, hq, q_len, kv_len), dtype=query.dtype, device=query.device)
 
     def strides(t):  # the stride of a dimension of one is never used and may be anything
-        return [t.stride(i) if t.shape[i] > 1 else 0 for i in range(3)]
+        (tb, th, tn, _), (sb, sh, sn, _) = t.shape, t.stride()
+        return sb if tb > 1 else 0, sh if th > 1 else 0, sn if tn > 1 else 0
 
-    with torch.cuda.device(query.device):
+    with _hip.on_device(query.device):
         _hip.check(_hip.load().mx_prefill_attn(
             query.data_ptr(), *strides(query), key.data_ptr(), *strides(key), value.data_ptr(), *strides(value), b, hq,
             hkv, q_len, kv_len, d, float(scaling), out.data_ptr(), weights.data_ptr(), _DTYPE_FLAGS[query.dtype],

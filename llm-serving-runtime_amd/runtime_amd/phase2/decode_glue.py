@@ -138,23 +138,26 @@ def kv_append(k_layer: torch.Tensor, v_layer: torch.Tensor, block_tables: torch.
         raise ValueError("kv_append supports fp16 or bf16 states and pools of the same dtype")
     b, hkv, t, d = key_states.shape
     nb, hkv_p, bs, d_p = k_layer.shape
-    if (hkv, d) != (hkv_p, d_p) or k_layer.stride() != v_layer.stride():
+    pool_strides = k_layer.stride()
+    if (hkv, d) != (hkv_p, d_p) or pool_strides != v_layer.stride():
         raise ValueError("states do not match the pool layout")
-    if k_layer.stride(3) != 1 or k_layer.stride(2) != d:
+    if pool_strides[3] != 1 or pool_strides[2] != d:
         raise ValueError("pool layer views must be contiguous within a (block, kv-head) run")
-    if key_states.stride(3) != 1 or value_states.stride() != key_states.stride():
+    strides = key_states.stride()
+    if strides[3] != 1 or value_states.stride() != strides:
         key_states = key_states.contiguous()
         value_states = value_states.contiguous()
+        strides = key_states.stride()
     tables = _i32(block_tables, dev)
     if tables.dim() != 2 or tables.shape[0] != b:
         raise ValueError("block_tables must be [B, max_blocks]")
-    starts = _i32(start_pos.reshape(-1), dev)
+    starts = _i32(start_pos if start_pos.dim() == 1 else start_pos.reshape(-1), dev)
     used = _used_ptr(used_blocks, nb, dev)
     lib = _hip.load()
     _hip.check(lib.mx_kv_append(
-        key_states.data_ptr(), value_states.data_ptr(), key_states.stride(0), key_states.stride(1),
-        key_states.stride(2), b, t, hkv, d, tables.data_ptr(), tables.stride(0), int(tables.shape[1]),
-        starts.data_ptr(), k_layer.data_ptr(), v_layer.data_ptr(), k_layer.stride(0), k_layer.stride(1), bs, nb,
+        key_states.data_ptr(), value_states.data_ptr(), strides[0], strides[1], strides[2], b, t, hkv, d,
+        tables.data_ptr(), tables.stride(0), tables.shape[1], starts.data_ptr(), k_layer.data_ptr(),
+        v_layer.data_ptr(), pool_strides[0], pool_strides[1], bs, nb,
         err.data_ptr() if err is not None else None, used, _hip.stream_handle(dev)), "mx_kv_append")
 
 
@@ -167,12 +170,14 @@ def kv_gather(k_layer: torch.Tensor, v_layer: torch.Tensor, block_tables: torch.
     nb, hkv, bs, d = k_layer.shape
     tables = _i32(block_tables, dev)
     b = int(tables.shape[0])
-    k, v = (torch.empty(b, hkv, tokens, d, dtype=k_layer.dtype, device=dev) for _ in range(2))
+    k = torch.empty((b, hkv, tokens, d), dtype=k_layer.dtype, device=dev)
+    v = torch.empty_like(k)
     lens = _i32(seq_lens.reshape(-1), dev) if seq_lens is not None else None
-    _hip.check(_hip.load().mx_kv_gather(
-        k_layer.data_ptr(), v_layer.data_ptr(), k_layer.stride(0), k_layer.stride(1), tables.data_ptr(),
-        tables.stride(0), int(tables.shape[1]), lens.data_ptr() if lens is not None else None, b, tokens, hkv, d, bs, nb,
-        k.data_ptr(), v.data_ptr(), None, _hip.stream_handle(dev)), "mx_kv_gather")
+    with _hip.on_device(dev):
+        _hip.check(_hip.load().mx_kv_gather(
+            k_layer.data_ptr(), v_layer.data_ptr(), k_layer.stride(0), k_layer.stride(1), tables.data_ptr(),
+            tables.stride(0), int(tables.shape[1]), lens.data_ptr() if lens is not None else None, b, tokens, hkv, d, bs,
+            nb, k.data_ptr(), v.data_ptr(), None, _hip.stream_handle(dev)), "mx_kv_gather")
     return k, v
 
 

@@ -103,28 +103,23 @@ def int8_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, bias
     n = int(out_features)
     if packed.numel() != n * k:
         raise ValueError(f"packed weight has {packed.numel()} bytes, expected {n}x{k}")
-    lead = x.shape[:-1]
-    x2 = x.reshape(-1, k)
-    if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
+    rows = x.dim() == 2
+    x2 = x if rows else x.reshape(-1, k)
+    xs, unit = x2.stride()
+    if unit != 1 or xs % 8 != 0 or x2.data_ptr() % 16 != 0:
         x2 = x2.contiguous()
-    m = int(x2.shape[0])
-    if out is None:
-        y = torch.empty((m, n), dtype=torch.float16, device=x.device)
-    else:
-        y = out.view(m, n)
-    if m == 0:
-        return y.view(*lead, n)
-    lib = _hip.load()
-    ws_ptr, ws_bytes = _workspace(x.device, int(lib.mx_w8a16_workspace_bytes(m, n, k)))
-    _hip.check(
-        lib.mx_w8a16_linear(
-            x2.data_ptr(), m, k, x2.stride(0), packed.data_ptr(), scale.data_ptr(),
-            bias.data_ptr() if bias is not None else None, y.data_ptr(), n, y.stride(0),
-            ws_ptr, ws_bytes, _hip.stream_handle(x.device),
-        ),
-        "mx_w8a16_linear",
-    )
-    return y.view(*lead, n)
+        xs = x2.stride(0)
+    m = x2.shape[0]
+    device = x.device
+    y = torch.empty((m, n), dtype=torch.float16, device=device) if out is None else out.view(m, n)
+    if m != 0:
+        ws_ptr, ws_bytes = _workspace(device, _hip.linear_workspace_bytes(m, n, k))
+        rc = _hip.load().mx_w8a16_linear(
+            x2.data_ptr(), m, k, xs, packed.data_ptr(), scale.data_ptr(), bias.data_ptr() if bias is not None else None,
+            y.data_ptr(), n, y.stride(0), ws_ptr, ws_bytes, _hip.stream_handle(device))
+        if rc != _hip.MX_OK:
+            _hip.check(rc, "mx_w8a16_linear")
+    return y if rows else y.view(*x.shape[:-1], n)
 
 
 def linear_splits(m: int, n: int, k: int) -> int:

@@ -100,7 +100,7 @@ _ws_lock = threading.Lock()
 
 
 def _workspace(device: torch.device, key: tuple) -> tuple[torch.Tensor, int]:
-    nbytes = int(_hip.load().mx_paged_attn_workspace_bytes(*key))
+    nbytes = _hip.attn_workspace_bytes(*key)
     full_key = (device, *key)
     ws = _workspaces.get(full_key)
     if ws is None:
@@ -143,45 +143,44 @@ def _decode(query: torch.Tensor, k_layer: torch.Tensor, v_layer: torch.Tensor, b
     if query.dtype not in _DTYPE_FLAGS or k_layer.dtype != query.dtype or v_layer.dtype != query.dtype:
         raise ValueError(f"HIP paged decode supports fp16 or bf16 query and pool of one dtype, got "
                          f"{query.dtype}/{k_layer.dtype}/{v_layer.dtype}")
-    nb, hkv, bs, dk = k_layer.shape
-    if tuple(v_layer.shape) != tuple(k_layer.shape) or v_layer.stride() != k_layer.stride():
+    shape, pool_strides = k_layer.shape, k_layer.stride()
+    nb, hkv, bs, dk = shape
+    if v_layer.shape != shape or v_layer.stride() != pool_strides:
         raise ValueError("K and V layer views must have the same shape and strides")
     if dk != d:
         raise ValueError(f"head_dim mismatch: query {d} vs pool {dk}")
     if hkv * num_kv_groups != hq:
         raise ValueError(f"num_heads {hq} != num_kv_heads {hkv} * num_kv_groups {num_kv_groups}")
-    if k_layer.stride(3) != 1 or k_layer.stride(2) != d:
+    if pool_strides[3] != 1 or pool_strides[2] != d:
         raise ValueError("pool layer views must be contiguous within a (block, kv-head) run")
     if query.stride(3) != 1:
         query = query.contiguous()
+    device = query.device
     if block_tables.dim() != 2 or block_tables.shape[0] != bsz:
         raise ValueError("block_tables must be [B, max_blocks]")
-    if block_tables.dtype != torch.int32 or block_tables.stride(1) != 1 or block_tables.device != query.device:
-        block_tables = block_tables.to(device=query.device, dtype=torch.int32).contiguous()
-    if seq_lens.dtype != torch.int32 or seq_lens.device != query.device or not seq_lens.is_contiguous():
-        seq_lens = seq_lens.to(device=query.device, dtype=torch.int32).contiguous()
-    max_blocks = int(block_tables.shape[1])
+    if block_tables.dtype != torch.int32 or block_tables.stride(1) != 1 or block_tables.device != device:
+        block_tables = block_tables.to(device=device, dtype=torch.int32).contiguous()
+    if seq_lens.dtype != torch.int32 or seq_lens.device != device or not seq_lens.is_contiguous():
+        seq_lens = seq_lens.to(device=device, dtype=torch.int32).contiguous()
+    max_blocks = block_tables.shape[1]
     if out is None:
-        out = torch.empty((bsz, hq, 1, d), dtype=query.dtype, device=query.device)
+        out = torch.empty((bsz, hq, 1, d), dtype=query.dtype, device=device)
     elif (tuple(out.shape) != (bsz, hq, 1, d) or out.dtype != query.dtype or out.stride(3) != 1
-          or out.device != query.device):
+          or out.device != device):
         raise ValueError("out must be a [B, heads, 1, dim] tensor of the query dtype with unit inner stride")
     if bsz == 0:
         return out
     key = (bsz, hq, hkv, d, max_blocks, bs, _CHUNK_TOKENS)
-    ws, nbytes = _workspace(query.device, key)
-    lib = _hip.load()
-    _hip.check(
-        lib.mx_paged_attn_decode(
-            query.data_ptr(), query.stride(0), query.stride(1), k_layer.data_ptr(), v_layer.data_ptr(),
-            k_layer.stride(0), k_layer.stride(1), block_tables.data_ptr(), block_tables.stride(0), max_blocks,
-            seq_lens.data_ptr(), bsz, hq, hkv, d, bs, nb, float(scaling), out.data_ptr(), out.stride(0),
-            out.stride(1), ws.data_ptr(), nbytes, _CHUNK_TOKENS,
-            _DTYPE_FLAGS[query.dtype] | (MX_PA_SHARED_BLOCKS if shared_blocks else 0) | plan,
-            _hip.stream_handle(query.device),
-        ),
-        "mx_paged_attn_decode",
-    )
+    ws, nbytes = _workspace(device, key)
+    q_sb, q_sh, _, _ = query.stride()
+    o_sb, o_sh, _, _ = out.stride()
+    rc = _hip.load().mx_paged_attn_decode(
+        query.data_ptr(), q_sb, q_sh, k_layer.data_ptr(), v_layer.data_ptr(), pool_strides[0], pool_strides[1],
+        block_tables.data_ptr(), block_tables.stride(0), max_blocks, seq_lens.data_ptr(), bsz, hq, hkv, d, bs, nb,
+        float(scaling), out.data_ptr(), o_sb, o_sh, ws.data_ptr(), nbytes, _CHUNK_TOKENS,
+        _DTYPE_FLAGS[query.dtype] | (MX_PA_SHARED_BLOCKS if shared_blocks else 0) | plan, _hip.stream_handle(device))
+    if rc != _hip.MX_OK:
+        _hip.check(rc, "mx_paged_attn_decode")
     return out
 
 

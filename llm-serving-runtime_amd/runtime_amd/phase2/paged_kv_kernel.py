@@ -178,13 +178,13 @@ class GpuKVBlockPool:
         """Per-layer K blocks: ``[num_blocks, num_kv_heads, block_size, head_dim]``."""
         self._ensure_pools()
         assert self._k_pool is not None
-        return self._k_pool[layer_idx]
+        return self._k_pool.select(0, layer_idx)
 
     def v_layer_view(self, layer_idx: int) -> torch.Tensor:
         """Per-layer V blocks: ``[num_blocks, num_kv_heads, block_size, head_dim]``."""
         self._ensure_pools()
         assert self._v_pool is not None
-        return self._v_pool[layer_idx]
+        return self._v_pool.select(0, layer_idx)
 
     def write_tokens(self, layer_idx: int, block_ids: list[int], start_pos: int, key_states: torch.Tensor,
                      value_states: torch.Tensor) -> None:
@@ -233,8 +233,10 @@ class GpuKVBlockPool:
         if device.type == "cuda":
             from .decode_glue import kv_append
 
-            kv_append(k_layer, v_layer, block_tables, start_positions, key_states.to(self.dtype),
-                      value_states.to(self.dtype), err=self._write_err, used_blocks=self._used_map)
+            if key_states.dtype != self.dtype or value_states.dtype != self.dtype:
+                key_states, value_states = key_states.to(self.dtype), value_states.to(self.dtype)
+            kv_append(k_layer, v_layer, block_tables, start_positions, key_states, value_states, err=self._write_err,
+                      used_blocks=self._used_map)
             if self.sync_write_checks and not torch.cuda.is_current_stream_capturing():
                 self.check_write_errors()
             return
