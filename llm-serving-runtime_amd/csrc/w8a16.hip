@@ -766,13 +766,11 @@ static bool use_m_split(int MT, int NT, int KT) {
     return MT >= 6 || (MT == 4 && KT / big_splits(NT, KT) >= kMwMinRangeTiles);
 }
 
-// gate||up (never split) goes to the many-row launch above 128 rows, and at 65-128 rows where the
-// M-split shape would leave more than half of the CUs without a workgroup: the Qwen2-0.5B gate||up
-// (76 workgroups) at 128 rows 13.9 -> 10.2 us on MI355X; the Llama-3-8B one (224 workgroups) takes 43
-// us here and 44-46 there.
-static bool gateup_takes_rows(int64_t M, int NT) {
-    return M > kMaxRows || (M > 64 && ceil_div(NT, kBigTiles) <= kBigGrid / 2);
-}
+// gate||up (never split) goes to the many-row launch above 64 rows: against the M-split shape, 28672 x
+// 4096 at 65 / 96 / 128 rows 45.6 / 42.7 / 48.7 -> 37.5 / 35.3 / 43.5 us, 11264 x 2048 at 100 rows 17.8 ->
+// 14.9, 9728 x 896 at 128 rows 11.7 -> 9.8 (MI355X). At 64 rows and below the 4-wave and wide shapes of this
+// file run it.
+constexpr int kGateupMaxRows = 64;
 
 static Plan plan_for(int M, int NT, int KT) {
     Plan pl{};
@@ -1272,19 +1270,19 @@ extern "C" int mx_w8a16_gateup_swiglu(const uint16_t* x, int64_t M, int64_t K, i
     const int NT = (int)(2 * I / w8a16::kTileN), KT = (int)(K / w8a16::kTileK);
     if ((int64_t)NT * w8a16::kTileN != 2 * I || K * 64 > 0x7fffffff)
         return fail(MX_ERR_UNSUPPORTED, "mx_w8a16_gateup_swiglu: bad shape");
-    // The many-row launch, or at most kMaxRows rows: the VALU GEMV where mx_w8a16_linear
+    // The many-row launch, or at most 64 rows at a time: the VALU GEMV where mx_w8a16_linear
     // would take it (M <= 4 on shapes that split), else one unsplit MFMA launch, also where
     // mx_w8a16_linear would split K: the epilogue needs the whole sum, and on such (small)
     // shapes one launch without K split costs less than a split launch plus a SwiGLU launch
     // (the Qwen2-0.5B MLP at batch 16).
     hipStream_t st = as_stream(stream);
-    if (w8a16::gateup_takes_rows(M, NT) && w8a16::rows_fit(M, x_stride, NT)) {
+    if (M > w8a16::kGateupMaxRows && w8a16::rows_fit(M, x_stride, NT)) {
         w8a16::launch_rows(true, w8a16::plan_rows(M, NT, KT, 0), x, x_stride, (int)M, packed, scale, bias, y, y_stride,
                            NT, KT, nullptr, st);
         return check_launch("mx_w8a16_gateup_swiglu");
     }
-    for (int64_t m0 = 0; m0 < M; m0 += w8a16::kMaxRows) {
-        const int mc = (int)(M - m0 < w8a16::kMaxRows ? M - m0 : w8a16::kMaxRows);
+    for (int64_t m0 = 0; m0 < M; m0 += w8a16::kGateupMaxRows) {
+        const int mc = (int)(M - m0 < w8a16::kGateupMaxRows ? M - m0 : w8a16::kGateupMaxRows);
         const uint16_t* xc = x + m0 * x_stride;
         uint16_t* yc = y + m0 * y_stride;
         const w8a16::Plan pl = w8a16::plan_for(mc, NT, KT);
@@ -1296,9 +1294,7 @@ extern "C" int mx_w8a16_gateup_swiglu(const uint16_t* x, int64_t M, int64_t K, i
             case 1: w8a16::launch_mfma<1, false, true>(xc, x_stride, mc, packed, scale, bias, yc, y_stride, NT, KT, 1, 1, nullptr, st); break;
             case 2: w8a16::launch_mfma<2, false, true>(xc, x_stride, mc, packed, scale, bias, yc, y_stride, NT, KT, 1, 1, nullptr, st); break;
             case 3: w8a16::launch_mfma<3, false, true>(xc, x_stride, mc, packed, scale, bias, yc, y_stride, NT, KT, 1, 1, nullptr, st); break;
-            case 4: w8a16::launch_mfma<4, false, true>(xc, x_stride, mc, packed, scale, bias, yc, y_stride, NT, KT, 1, 1, nullptr, st); break;
-            case 6: w8a16::launch_mfma<6, false, true>(xc, x_stride, mc, packed, scale, bias, yc, y_stride, NT, KT, 1, 1, nullptr, st); break;
-            default: w8a16::launch_mfma<8, false, true>(xc, x_stride, mc, packed, scale, bias, yc, y_stride, NT, KT, 1, 1, nullptr, st); break;
+            default: w8a16::launch_mfma<4, false, true>(xc, x_stride, mc, packed, scale, bias, yc, y_stride, NT, KT, 1, 1, nullptr, st); break;
         }
     }
     return check_launch("mx_w8a16_gateup_swiglu");

@@ -7,8 +7,9 @@ namespace mx {
 namespace w8a16 {
 
 struct RowsPlan {
-    int MT;  // 16-row tiles per workgroup
-    int KS;  // k ranges; more than one writes fp32 partials [KS][M][N]
+    int MT;   // 16-row tiles per workgroup
+    int NPW;  // n-tiles per wave (4 waves per workgroup)
+    int KS;   // k ranges; more than one writes fp32 partials [KS][M][N]
 };
 
 // The plan of an M-row launch whose partials may take up to partial_bytes (0: no ranges).

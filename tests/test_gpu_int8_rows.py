@@ -1,4 +1,4 @@
-"""GPU: the many-row int8 GEMM (more than 128 rows, and gate||up at 65-128 rows on narrow shapes)
+"""GPU: the many-row int8 GEMM (more than 128 rows, and gate||up above 64 rows)
 against the product of the same quantized weights in float64.
 
 Bound: fp32 accumulation of K terms (K * 2^-24 of the sum of their magnitudes), then one rounding to
@@ -35,12 +35,15 @@ def _product(x, w, bias=None):
     return y, U * y.abs() + SUB + (x.shape[1] + 2) * 2.0**-24 * mag
 
 
-# Row tiles of 32, 64, 96 and 128 rows with remainders, n-tiles past the last one (N / 16 not a
-# multiple of 16), one k-tile, odd and even k-tile counts, and shapes that split K.
+# Every row tile (32, 64, 96, 128 rows) and both widths (128 and 256 channels) with remainders, n-tiles
+# past the last one, one k-tile, k-tile counts around the unrolled loops' 2, 3 and 12, and shapes that
+# split K.
 @pytest.mark.parametrize("m,n,k,bias", [
     (129, 1152, 896, True), (777, 1152, 896, True), (160, 4096, 4096, False), (256, 896, 4864, True),
     (1531, 4096, 1024, False), (2049, 4112, 192, True), (1000, 16, 64, False), (130, 272, 64, True),
     (385, 6144, 4096, False), (4096, 2048, 128, False), (191, 4096, 14336, False),
+    (256, 4096, 14336, False), (1531, 4096, 14336, False), (700, 28672, 832, True), (2048, 28672, 1600, False),
+    (130, 6144, 704, False), (140, 2048, 768, True), (150, 1024, 1600, False),
 ])
 def test_linear(m, n, k, bias):
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
@@ -77,7 +80,8 @@ def test_without_workspace_runs_in_one_range():
 
 @pytest.mark.parametrize("m,inter,k,bias", [
     (65, 4864, 896, False), (128, 4864, 896, True), (129, 4864, 896, False), (777, 1032, 192, True),
-    (2048, 14336, 256, False), (300, 14336, 4096, False), (150, 8, 64, False),
+    (2048, 14336, 256, False), (300, 14336, 4096, False), (150, 8, 64, False), (96, 14336, 4096, False),
+    (128, 14336, 4096, True), (66, 5632, 2048, False), (2000, 14336, 1088, False), (64, 4864, 896, False),
 ])
 def test_gateup(m, inter, k, bias):
     g = torch.Generator(device=DEV).manual_seed(m + inter + k)
