@@ -15,8 +15,8 @@
 // products), so each half k-tile's fragments and weights are made ready under the previous half's
 // products: 0.47-0.60 -> 0.43-0.53 us per k-tile for one workgroup of 32 or 64 rows x 256 channels, and
 // 0.25-0.34 us with 128 channels. Many are bound by the matrix cores together with what feeds them.
-// Llama-3-8B gate||up at 2048 rows: 646 -> 410 us (744 -> 1170 TFLOP/s; torch's fp16 product of that size
-// takes 418 us). The MFMAs and barriers alone take 272 us; without the dequant it would be 385, without
+// Llama-3-8B gate||up at 2048 rows: 646-668 -> 416-431 us (720-744 -> 1115-1155 TFLOP/s; torch's fp16
+// product of that size takes 418 us). The MFMAs and barriers alone take 272 us; without the dequant it would be 385, without
 // the weight loads 323-360, without the x loads 374. Loads two or three k-tiles ahead measured the
 // same, 8 waves per workgroup (128 x 512 or 256 x 256) 440-500 us: one barrier then holds the whole CU.
 #include "w8a16_rows.h"

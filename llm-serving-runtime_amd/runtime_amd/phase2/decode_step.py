@@ -38,7 +38,7 @@ Llama / Qwen2 style (pre-norm, rotate-half RoPE, GQA, SwiGLU, untied int8
 lm_head); :meth:`Int8DecodeModel.from_hf` loads the weights of an HF
 ``LlamaForCausalLM`` / ``Qwen2ForCausalLM``. The gate||up weight is stored
 with gate and up rows interleaved in groups of 8 (``gateup_interleave``), and
-one ``mx_w8a16_gateup_swiglu`` launch per 128 rows writes ``silu(g) * u``
+one ``mx_w8a16_gateup_swiglu`` launch writes ``silu(g) * u``
 whatever the batch: it never splits K (on shapes whose plain projection would,
 such as Qwen2-0.5B at batch 16, it runs unsplit), and at most 4 rows run on
 the VALU GEMV with the product in its own epilogue.
@@ -364,7 +364,7 @@ class Int8DecodeModel:
             add_rmsnorm(buf.mlp, weight, eps, residual=buf.h, out=buf.x, residual_out=buf.h)
 
     def _gate_up(self, buf: _Buffers, w, bsz: int, timers) -> None:
-        """act = silu(gate) * up from the interleaved gate||up weight, one launch per 128 rows."""
+        """act = silu(gate) * up from the interleaved gate||up weight, one launch."""
         packed, scale, n, bias = w
         ev = self._tick(timers, "gate_up")
         int8_gateup_swiglu(buf.x, packed, scale, bias, n // 2, out=buf.act)
