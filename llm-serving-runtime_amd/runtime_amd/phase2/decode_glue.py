@@ -168,14 +168,25 @@ def kv_gather(k_layer: torch.Tensor, v_layer: torch.Tensor, block_tables: torch.
     ids must be in the pool (a token of one that is not comes back zero)."""
     dev = k_layer.device
     nb, hkv, bs, d = k_layer.shape
+    strides = k_layer.stride()
+    if v_layer.shape != k_layer.shape or v_layer.stride() != strides or v_layer.dtype != k_layer.dtype:
+        raise ValueError("K and V layer views must have the same shape, strides and dtype")
+    if k_layer.dtype not in (torch.float16, torch.bfloat16):
+        raise ValueError(f"kv_gather supports fp16 or bf16 pools, got {k_layer.dtype}")
+    if strides[3] != 1 or strides[2] != d:
+        raise ValueError("pool layer views must be contiguous within a (block, kv-head) run")
+    if block_tables.dim() != 2:
+        raise ValueError("block_tables must be [B, max_blocks]")
+    b = int(block_tables.shape[0])
+    if seq_lens is not None and seq_lens.numel() != b:
+        raise ValueError(f"{b} block-table rows but {seq_lens.numel()} lengths")
     tables = _i32(block_tables, dev)
-    b = int(tables.shape[0])
     k = torch.empty((b, hkv, tokens, d), dtype=k_layer.dtype, device=dev)
     v = torch.empty_like(k)
     lens = _i32(seq_lens.reshape(-1), dev) if seq_lens is not None else None
     with _hip.on_device(dev):
         _hip.check(_hip.load().mx_kv_gather(
-            k_layer.data_ptr(), v_layer.data_ptr(), k_layer.stride(0), k_layer.stride(1), tables.data_ptr(),
+            k_layer.data_ptr(), v_layer.data_ptr(), strides[0], strides[1], tables.data_ptr(),
             tables.stride(0), int(tables.shape[1]), lens.data_ptr() if lens is not None else None, b, tokens, hkv, d, bs,
             nb, k.data_ptr(), v.data_ptr(), None, _hip.stream_handle(dev)), "mx_kv_gather")
     return k, v

@@ -313,6 +313,8 @@ class GpuKVBlockPool:
         max_seq = max(lens) if lens else 0
         if max_seq <= 0:
             raise ValueError("seq_len must be positive")
+        if len(lens) < batch_size:
+            raise IndexError(f"{batch_size} block-table rows but {len(lens)} lengths")
         if self._gathers_on_device():
             for row, n in zip(block_tables.tolist(), lens):
                 if n <= 0:
@@ -321,7 +323,7 @@ class GpuKVBlockPool:
                 if n_logical > len(row):
                     raise IndexError("block table underrun during gather")
                 self._touch_ids([int(i) for i in row[:n_logical]])
-            return self._gather_table(layer_idx, block_tables, max_seq, seq_lens)
+            return self._gather_table(layer_idx, block_tables, max_seq, seq_lens[:batch_size])
         s = self.shape
         keys = torch.zeros(batch_size, s.num_kv_heads, max_seq, s.head_dim, device=self.device, dtype=self.dtype)
         values = torch.zeros_like(keys)

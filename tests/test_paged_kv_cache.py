@@ -9,11 +9,14 @@ pool oracle.
 
 from __future__ import annotations
 
+import contextlib
+
 import pytest
 import torch
 
 from oracle import kv_pool as okv
 from oracle import model as om
+from runtime_amd.phase2 import _hip
 from runtime_amd.phase2.hf_decode import enable_block_paged_attention, prefill_request
 from runtime_amd.phase2.paged_attention_hip import get_paged_decode_batch_metadata, set_paged_decode_batch_metadata
 from runtime_amd.phase2.paged_kv_cache import BlockPagedBatchCache, BlockPagedCache
@@ -206,3 +209,63 @@ def test_greedy_decode_plumbing_with_oracle_attention():
         assert tokens[b].tolist() == ref_tokens.tolist()
     with pytest.raises(ValueError):
         greedy_decode(model, pool, prompts[:1], [[1]], steps)
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """Pools said to be on a device, with the gather's launch recorded in place of done: the checks
+    ahead of it run on the host."""
+    seen = []
+
+    class _Lib:
+        def mx_kv_gather(self, *args):
+            seen.append(args)
+            return 0
+
+    monkeypatch.setattr(_hip, "load", lambda: _Lib())
+    monkeypatch.setattr(_hip, "stream_handle", lambda device: 0)
+    monkeypatch.setattr(_hip, "on_device", lambda device: contextlib.nullcontext())
+    return seen
+
+
+def _device_pool(monkeypatch, num_blocks=8):
+    pool = GpuKVBlockPool(num_blocks=num_blocks, block_size_tokens=BS, num_layers=1, num_kv_heads=HKV, head_dim=D,
+                          dtype=torch.float16, device="cpu")
+    pool._ensure_pools()
+    monkeypatch.setattr(pool, "_gathers_on_device", lambda: True)
+    return pool
+
+
+@pytest.mark.parametrize("rows,lens,error", [
+    ([[0, 1], [2, 3], [4, 5]], [5, 8], IndexError),      # fewer lengths than rows
+    ([[0, 1], [2, 3], [4, 8]], [5, 8, 8], IndexError),   # a block outside the pool in the last row
+    ([[0, 1], [2, 3]], [5, 9], IndexError),              # a table with too few blocks
+    ([[0, 1], [2, 3]], [5, 0], ValueError),              # an empty row
+    ([[0, 1], [2, 3]], [5, 8], None),
+    ([[0, 1], [2, 3]], [5, 8, 3], None),                 # lengths past the rows are not read
+])
+def test_batched_gather_checks_every_row_before_the_launch(monkeypatch, launches, rows, lens, error):
+    pool = _device_pool(monkeypatch)
+    tables, lengths = torch.tensor(rows, dtype=torch.int32), torch.tensor(lens, dtype=torch.int32)
+    if error is not None:
+        with pytest.raises(error):
+            pool.gather_layer_batch(0, tables, lengths)
+        assert not launches
+        return
+    keys, values = pool.gather_layer_batch(0, tables, lengths)
+    assert keys.shape == values.shape == (len(rows), HKV, max(lens), D) and len(launches) == 1
+
+
+def test_kv_gather_refuses_shapes_the_launch_would_read_past(launches):
+    from runtime_amd.phase2.decode_glue import kv_gather
+
+    k = torch.zeros(8, HKV, BS, D, dtype=torch.float16)
+    tables, lens = torch.zeros(3, 2, dtype=torch.int32), torch.ones(3, dtype=torch.int32)
+    for args in ((k, k, tables, 4, lens[:2]), (k, k, tables[0], 4, None), (k, k[:4], tables, 4, lens),
+                 (k, k.transpose(0, 1).contiguous().transpose(0, 1), tables, 4, lens), (k[..., :16], k[..., :16], tables, 4, lens),
+                 (k.float(), k.float(), tables, 4, lens), (k, k.bfloat16(), tables, 4, lens)):
+        with pytest.raises(ValueError):
+            kv_gather(*args)
+    assert not launches
+    kv_gather(k, k, tables, 4, lens)
+    assert len(launches) == 1
