@@ -116,22 +116,16 @@ class BlockPagedLayer(CacheLayerMixin):
             return key_states, value_states
 
         set_paged_decode_batch_metadata(None)
-        return self._rows(start, table, key_states, value_states)
+        return self._rows(table)
 
-    def _rows(self, start: int, table: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor
-              ) -> tuple[torch.Tensor, torch.Tensor]:
-        """K and V of the row's tokens after a prefill write, ``pool.gather_layer``'s values: the new
-        states themselves when they are the whole row in the pool's dtype and every block has a place
-        of its own (nothing to read back), else gathered in one launch over the row's device table."""
+    def _rows(self, table: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        """K and V of the row's tokens after a prefill write, ``pool.gather_layer``'s values in tensors of
+        their own (never the caller's states, which it may refill), in one launch over the row's device
+        table where there is one."""
         pool = self.pool
         if not pool._gathers_on_device() or table.dtype != torch.int32 or table.device.type != "cuda":
             return pool.gather_layer(self.layer_idx, self._block_ids, self._seq_len)
-        ids = [int(b) for b in self._block_ids[: -(-self._seq_len // pool.block_size_tokens)]]
-        distinct = pool._touch_ids(ids)
-        if start == 0 and len(distinct) == len(ids) and all(
-                t.dtype == pool.dtype and t.device == table.device and not t.requires_grad
-                for t in (key_states, value_states)):
-            return key_states, value_states
+        pool._touch_ids([int(b) for b in self._block_ids[: -(-self._seq_len // pool.block_size_tokens)]])
         return pool._gather_table(self.layer_idx, table, self._seq_len)
 
     def get_mask_sizes(self, query_length: int) -> tuple[int, int]:

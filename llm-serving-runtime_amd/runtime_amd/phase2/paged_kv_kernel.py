@@ -159,15 +159,14 @@ class GpuKVBlockPool:
     def _touch_blocks(self, physical_ids: torch.Tensor) -> None:
         self._touch_ids(physical_ids.unique().tolist())
 
-    def _touch_ids(self, ids: list[int]) -> set[int]:
-        """:meth:`_touch_block` of every id; the distinct ones."""
+    def _touch_ids(self, ids: list[int]) -> None:
+        """:meth:`_touch_block` of every id."""
         distinct = set(ids)
         if distinct and (min(distinct) < 0 or max(distinct) >= self.shape.num_blocks):
             for physical in ids:  # raises at the first id out of range
                 self._touch_block(int(physical))
         self._used_blocks |= distinct
         self._peak_allocated_blocks = max(self._peak_allocated_blocks, len(self._used_blocks))
-        return distinct
 
     def _gathers_on_device(self) -> bool:
         """Whether rows come out of the pool by ``mx_kv_gather``: 16-bit elements in 16-byte chunks."""

@@ -117,3 +117,20 @@ def test_prefill_update_with_a_block_outside_the_pool_raises():
     k = torch.randn(1, 2, 20, 64, device=DEV).half()
     with pytest.raises(IndexError):
         layer.update(k, k)
+
+
+@pytest.mark.parametrize("start,new", [(0, 20), (16, 9)])
+def test_prefill_update_returns_rows_of_its_own(start, new):
+    """What ``update`` returned stays as it was when the caller refills the buffers it passed."""
+    from runtime_amd.phase2.paged_kv_cache import BlockPagedLayer
+
+    pool = _filled_pool("interleaved", 16, 2, 16, 64, 1, seed=6)
+    layer = BlockPagedLayer(pool, 0)
+    layer.set_block_ids([3, 9])
+    layer.set_seq_length(start)
+    gen = torch.Generator().manual_seed(7)
+    k, v = (torch.randn(1, 2, new, 64, generator=gen).half().to(DEV) for _ in range(2))
+    got = layer.update(k, v)
+    want = k.clone(), v.clone()
+    k.fill_(1.0), v.fill_(2.0)
+    assert torch.equal(got[0][:, :, start:], want[0]) and torch.equal(got[1][:, :, start:], want[1])
