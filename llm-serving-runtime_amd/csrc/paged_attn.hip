@@ -691,7 +691,10 @@ struct PartVec<8> {
 
 // One batch of the online log-sum-exp over a lane's pieces: the UB pieces' (m, l) and normalised
 // outputs, of which the first cnt are real (the rest masked). Branch-free, so that loads issued before
-// it are not sunk behind anything. mg, l and a stay the lane's own (over its pieces so far).
+// it are not sunk behind anything. mg, l and a stay the lane's own (over its pieces so far). A piece
+// with m = -inf weighs 0: its l is 0 (every block of it skipped), or NaN where its scores were, and
+// that NaN goes on into l, also when it is the lane's only piece: the head's output is then 0, never
+// the attention over the other pieces alone.
 template <int UB, int VD, bool BF16>
 __device__ __forceinline__ void merge_step(const float2 (&ml)[UB], const typename PartVec<VD>::type (&av)[UB], int cnt,
                                            float& mg, float& l, float (&a)[VD]) {
@@ -699,9 +702,9 @@ __device__ __forceinline__ void merge_step(const float2 (&ml)[UB], const typenam
     float mc = kNegInf;
 #pragma unroll
     for (int u = 0; u < UB; ++u) mc = u < cnt ? fmaxf(mc, ml[u].x) : mc;
-    const float mn = fmaxf(mg, mc);
-    const bool any = mn != kNegInf;  // false while every tile so far was skipped
-    const float r = any ? __builtin_amdgcn_exp2f(mg - mn) : 1.0f;
+    mc = fmaxf(mg, mc);
+    const float mn = mc != kNegInf ? mc : 0.0f;  // the reference point: finite while every maximum is -inf
+    const float r = __builtin_amdgcn_exp2f(mg - mn);
     l *= r;
 #pragma unroll
     for (int e = 0; e < VD; ++e) a[e] *= r;
@@ -709,7 +712,7 @@ __device__ __forceinline__ void merge_step(const float2 (&ml)[UB], const typenam
     // away, never multiplied by 0.
 #pragma unroll
     for (int u = 0; u < UB; ++u) {
-        const bool v = u < cnt && any;
+        const bool v = u < cnt;
         const float wgt = __builtin_amdgcn_exp2f(ml[u].x - mn) * ml[u].y;
         l = v ? l + wgt : l;
 #pragma unroll
@@ -718,7 +721,7 @@ __device__ __forceinline__ void merge_step(const float2 (&ml)[UB], const typenam
             a[e] = v ? t : a[e];
         }
     }
-    mg = any ? mn : mg;
+    mg = mc;
 }
 
 // U: slots per segment window and partials loaded per memory round trip (Params::seg_slots).
@@ -765,7 +768,7 @@ __global__ __launch_bounds__(G * 64) void decode_merge_kernel(Params p) {
         }
         merge_step<UB, VD, BF16>(ml, av, mine - i0 / kMergeGroups, mg, l, a);
     }
-    // The four lanes of a dim group: rescale to the common maximum and add.
+    // The four lanes of a dim group: rescale to the common maximum and add (a NaN l stays one: NaN * 0).
     const float mx = xor_max_16_32(mg);
     const float r = mg != -__builtin_huge_valf() ? __builtin_amdgcn_exp2f(mg - mx) : 0.0f;
     l = xor_sum_16_32(l * r);

@@ -10,6 +10,7 @@ GQA 1..8, D 64/128, block size 16/32, split granularities).
 from __future__ import annotations
 
 import math
+import sys
 
 import numpy as np
 import pytest
@@ -567,3 +568,28 @@ def test_interleaved_pool_layout_is_bit_identical(d, bs, grp):
     assert torch.equal(split, inter)
     _check(inter, oracle_out(q, ki, vi, tables, lens, scale, grp))
     assert workspace_error_flag() == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,pieces,bad", [(64, 4, 1), (128, 4, 3), (64, 7, 5), (128, 20, 18)])
+def test_a_piece_of_nan_scores_is_not_dropped_by_the_merge(monkeypatch, dtype, d, pieces, bad):
+    """Ranges of 64 tokens: piece ``bad`` of kv-head 0 has only NaN scores, the others are ordinary.
+    The heads of kv-head 0 come back 0 (a NaN denominator), never as attention over the other
+    pieces; kv-head 1 keeps its bits."""
+    monkeypatch.setattr(sys.modules[paged_attention_decode_batched.__module__], "_CHUNK_TOKENS", 64)
+    bs, hkv, grp, tokens = 16, 2, 3, 64 * pieces
+    g = torch.Generator().manual_seed(d + pieces)
+    pool = GpuKVBlockPool(num_blocks=tokens // bs, block_size_tokens=bs, num_layers=1, num_kv_heads=hkv, head_dim=d,
+                          dtype=dtype, device="cuda")
+    for view in (pool.k_layer_view(0), pool.v_layer_view(0)):
+        view.copy_(torch.randn(view.shape, generator=g))
+    q = torch.randn(1, hkv * grp, 1, d, generator=g).to("cuda", dtype)
+    meta = PagedDecodeBatchMetadata(
+        pool=pool, layer_idx=0, block_tables=torch.arange(tokens // bs, dtype=torch.int32, device="cuda").view(1, -1),
+        seq_lens=torch.tensor([tokens], dtype=torch.int32, device="cuda"))
+    clean = paged_attention_decode_batched(q, meta, grp, d ** -0.5)
+    pool.k_layer_view(0)[bad * 64 // bs:(bad + 1) * 64 // bs, 0] = float("nan")
+    got = paged_attention_decode_batched(q, meta, grp, d ** -0.5)
+    assert clean.isfinite().all()
+    assert (got[:, :grp] == 0).all()
+    assert torch.equal(got[:, grp:], clean[:, grp:])
