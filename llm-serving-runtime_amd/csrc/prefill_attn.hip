@@ -324,9 +324,10 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(Params p) {
     __syncthreads();
 
     // The weights of the tokens past the wave's last tile: 0, or NaN where the row's own are (the
-    // softmax of a row with a NaN or an infinite score is NaN at its masked tokens as well). Whole
-    // lines that nothing here reads again: stored with the streaming policy, 113 -> 101 us for the
-    // Llama-3-8B heads at 2048 tokens. The weights' own stores, half a line each, lost by it (121).
+    // softmax of a row with a NaN or a +inf score, or with none above -inf, whose bias is +inf, is NaN
+    // at its masked tokens as well). Whole lines that nothing here reads again: stored with the
+    // streaming policy, 113 -> 101 us for the Llama-3-8B heads at 2048 tokens. The weights' own stores,
+    // half a line each, lost by it (121).
     const int zero0 = (wave_end + kTok - 1) / kTok * kTok;
     if (zero0 < p.S) {
         constexpr uint32_t kNan = BF16 ? 0x7fc07fc0u : 0x7e007e00u;
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(Params p) {
                 const int row = row0 + 16 * t + i;
                 if (row >= p.P) break;
                 const float bi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bias[t]), i));
-                const uint32_t w = bi != bi ? kNan : 0u;
+                const uint32_t w = __builtin_fabsf(bi) < __builtin_huge_valf() ? 0u : kNan;
                 const u32x4v fill{w, w, w, w};
                 for (int tok = zero0 + 8 * lane; tok < p.S; tok += 512) {
                     _Float16* dst = p.weights + (wrow + row) * p.S + tok;

@@ -115,3 +115,18 @@ def test_what_the_kernel_leaves_to_the_eager_chain():
     out, _ = bpa.block_paged_attention_forward(module, qg, k, k, None, 0.125)
     out.float().sum().backward()
     assert qg.grad is not None
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,s", [(64, 100), (128, 320), (64, 129)])
+def test_a_row_whose_visible_scores_are_all_minus_infinity_is_nan_everywhere(dtype, d, s):
+    g = torch.Generator().manual_seed(s)
+    q, k, v = (torch.randn(1, 2, s, d, generator=g).to(DEV, dtype) for _ in range(3))
+    module = SimpleNamespace(num_key_value_groups=1, training=False)
+    k[0, :, 0, 3] = -1.0
+    q[0, 1, 0, 3] = float("inf")  # row 0 sees token 0 alone: its score is -inf
+    base = bpa.block_paged_attention_forward(module, q[:, :1], k[:, :1], v[:, :1], None, 0.125)
+    out, weights = bpa.block_paged_attention_forward(module, q, k, v, None, 0.125)
+    assert weights[0, 1, 0].isnan().all() and out[0, 0, 1].isnan().all()
+    assert torch.equal(weights[0, :1], base[1][0]) and torch.equal(out[0, :, :1], base[0][0])
+    assert weights[0, 1, 1:].isfinite().all() and out[0, 1:, 1].isfinite().all()
