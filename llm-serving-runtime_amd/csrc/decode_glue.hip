@@ -110,7 +110,7 @@ struct GatherParams {
     int64_t bt_sb;
     int max_blocks;
     const int32_t* lens;  // NULL: every row has S tokens
-    int S, Hkv, D, bs, num_pool_blocks;
+    int B, S, Hkv, D, bs, num_pool_blocks;
     uint16_t* k_out;      // [B, Hkv, S, D]
     uint16_t* v_out;
     int32_t* err;
@@ -119,28 +119,32 @@ struct GatherParams {
 // K and V of whole rows out of the pool: blockIdx.y is one (row, kv-head), a thread copies one
 // 8-element chunk of one token of K and of V, so stores are contiguous and loads contiguous within
 // a block's run. Tokens past the row's length are zero. Bound by its bytes; the torch chain it
-// replaces (an index and a reshape copy for each of K and V) moved them twice.
+// replaces (an index and a reshape copy for each of K and V) moved them twice. A grid dimension
+// holds 65535 (row, kv-head) pairs; with more, a workgroup takes every gridDim.y-th.
+constexpr int kMaxGridY = 65535;
 __global__ __launch_bounds__(kThreads) void kv_gather_kernel(GatherParams p) {
     const int chunks = p.D >> 3;
     const int i = blockIdx.x * kThreads + threadIdx.x;
     const int t = i / chunks;
     if (t >= p.S) return;
     const int c = i - t * chunks;
-    const int b = blockIdx.y / p.Hkv, h = blockIdx.y - b * p.Hkv;
-    uint4 k{0, 0, 0, 0}, v{0, 0, 0, 0};
-    if (!p.lens || t < p.lens[b]) {
-        const int64_t src = slot_offset(p.bt, p.bt_sb, p.max_blocks, b, t, p.bs, p.num_pool_blocks, p.sblk, p.shead, h,
-                                        p.D);
-        if (src >= 0) {
-            k = ld16(p.k_pool + src + c * 8);
-            v = ld16(p.v_pool + src + c * 8);
-        } else if (p.err && c == 0) {
-            atomicOr(p.err, 1);
+    for (int row = blockIdx.y; row < p.B * p.Hkv; row += gridDim.y) {
+        const int b = row / p.Hkv, h = row - b * p.Hkv;
+        uint4 k{0, 0, 0, 0}, v{0, 0, 0, 0};
+        if (!p.lens || t < p.lens[b]) {
+            const int64_t src = slot_offset(p.bt, p.bt_sb, p.max_blocks, b, t, p.bs, p.num_pool_blocks, p.sblk,
+                                            p.shead, h, p.D);
+            if (src >= 0) {
+                k = ld16(p.k_pool + src + c * 8);
+                v = ld16(p.v_pool + src + c * 8);
+            } else if (p.err && c == 0) {
+                atomicOr(p.err, 1);
+            }
         }
+        const int64_t dst = ((int64_t)row * p.S + t) * p.D + c * 8;
+        st16(p.k_out + dst, k);
+        st16(p.v_out + dst, v);
     }
-    const int64_t dst = ((int64_t)blockIdx.y * p.S + t) * p.D + c * 8;
-    st16(p.k_out + dst, k);
-    st16(p.v_out + dst, v);
 }
 
 struct RopeAppendParams {
@@ -636,13 +640,15 @@ extern "C" int mx_kv_gather(const uint16_t* k_pool, const uint16_t* v_pool, int6
     if (Hkv <= 0 || D <= 0 || D % 8 || block_size <= 0 || max_blocks <= 0 || num_pool_blocks <= 0)
         return fail(MX_ERR_INVALID, "%s: need Hkv, max_blocks, block_size, pool > 0 and D %% 8 == 0 (Hkv=%d D=%d)", what,
                     Hkv, D);
-    if ((int64_t)B * Hkv > 65535 || (int64_t)S * (D / 8) > 0x7fffff00)
+    const int64_t rows = (int64_t)B * Hkv;
+    if (rows > 0x7fff0000 || (int64_t)S * (D / 8) > 0x7fffff00)
         return fail(MX_ERR_UNSUPPORTED, "%s: too many rows or tokens", what);
     if (kv_sblk % 8 || kv_shead % 8 || !glue::a16(k_pool) || !glue::a16(v_pool) || !glue::a16(k_out) || !glue::a16(v_out))
         return fail(MX_ERR_ALIGNMENT, "%s: pool and outputs need 16-byte aligned rows", what);
-    glue::GatherParams p{k_pool, v_pool, kv_sblk, kv_shead, block_tables, bt_sb, max_blocks, seq_lens, S, Hkv, D,
-                         block_size, num_pool_blocks, k_out, v_out, err};
-    const dim3 grid((unsigned)ceil_div((int64_t)S * (D / 8), glue::kThreads), (unsigned)(B * Hkv));
+    glue::GatherParams p{k_pool, v_pool, kv_sblk, kv_shead, block_tables, bt_sb, max_blocks, seq_lens, B, S, Hkv,
+                         D, block_size, num_pool_blocks, k_out, v_out, err};
+    const dim3 grid((unsigned)ceil_div((int64_t)S * (D / 8), glue::kThreads),
+                    (unsigned)(rows < glue::kMaxGridY ? rows : glue::kMaxGridY));
     hipLaunchKernelGGL(glue::kv_gather_kernel, grid, dim3(glue::kThreads), 0, as_stream(stream), p);
     return check_launch(what);
 }

@@ -123,7 +123,7 @@ class BlockPagedLayer(CacheLayerMixin):
         their own (never the caller's states, which it may refill), in one launch over the row's device
         table where there is one."""
         pool = self.pool
-        if not pool._gathers_on_device() or table.dtype != torch.int32 or table.device.type != "cuda":
+        if not pool._gathers_on_device(self._seq_len) or table.dtype != torch.int32 or table.device.type != "cuda":
             return pool.gather_layer(self.layer_idx, self._block_ids, self._seq_len)
         pool._touch_ids([int(b) for b in self._block_ids[: -(-self._seq_len // pool.block_size_tokens)]])
         return pool._gather_table(self.layer_idx, table, self._seq_len)

@@ -168,10 +168,11 @@ class GpuKVBlockPool:
         self._used_blocks |= distinct
         self._peak_allocated_blocks = max(self._peak_allocated_blocks, len(self._used_blocks))
 
-    def _gathers_on_device(self) -> bool:
-        """Whether rows come out of the pool by ``mx_kv_gather``: 16-bit elements in 16-byte chunks."""
+    def _gathers_on_device(self, tokens: int) -> bool:
+        """Whether rows of ``tokens`` come out of the pool by ``mx_kv_gather``: 16-bit elements in 16-byte
+        chunks, whose number in a row is a 32-bit index there."""
         return (self.device.type == "cuda" and self.dtype in (torch.float16, torch.bfloat16)
-                and self.shape.head_dim % 8 == 0)
+                and self.shape.head_dim % 8 == 0 and tokens * (self.shape.head_dim // 8) <= 0x7fffff00)
 
     def k_layer_view(self, layer_idx: int) -> torch.Tensor:
         """Per-layer K blocks: ``[num_blocks, num_kv_heads, block_size, head_dim]``."""
@@ -288,7 +289,7 @@ class GpuKVBlockPool:
         assert self._k_pool is not None and self._v_pool is not None
         ids_list = [int(b) for b in list(block_ids)[:n_logical]]
         self._touch_ids(ids_list)
-        if self._gathers_on_device():
+        if self._gathers_on_device(seq_len):
             table = torch.tensor([ids_list], dtype=torch.int32).to(self.device)
             return self._gather_table(layer_idx, table, seq_len)
         ids = torch.tensor(ids_list, device=self.device, dtype=torch.long)
@@ -314,7 +315,7 @@ class GpuKVBlockPool:
             raise ValueError("seq_len must be positive")
         if len(lens) < batch_size:
             raise IndexError(f"{batch_size} block-table rows but {len(lens)} lengths")
-        if self._gathers_on_device():
+        if self._gathers_on_device(max_seq):
             for row, n in zip(block_tables.tolist(), lens):
                 if n <= 0:
                     raise ValueError("seq_len must be positive")

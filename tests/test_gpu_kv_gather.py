@@ -134,3 +134,14 @@ def test_prefill_update_returns_rows_of_its_own(start, new):
     want = k.clone(), v.clone()
     k.fill_(1.0), v.fill_(2.0)
     assert torch.equal(got[0][:, :, start:], want[0]) and torch.equal(got[1][:, :, start:], want[1])
+
+
+def test_gather_of_more_rows_than_a_grid_dimension_holds():
+    pool = _filled_pool("interleaved", 16, 2, 4, 64, 1, seed=8)
+    rows = 40000  # 80000 (row, kv-head) pairs
+    tables = torch.arange(rows, dtype=torch.int32, device=DEV).remainder(16).view(-1, 1)
+    lens = torch.arange(rows, dtype=torch.int32, device=DEV).remainder(4) + 1
+    got = pool.gather_layer_batch(0, tables, lens)
+    seen = (torch.arange(4, device=DEV)[None] < lens[:, None])[:, None, :, None]
+    for out, view in zip(got, (pool.k_layer_view(0), pool.v_layer_view(0))):
+        assert torch.equal(out, torch.where(seen, view[tables[:, 0].long()], 0))

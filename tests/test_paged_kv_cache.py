@@ -232,7 +232,7 @@ def _device_pool(monkeypatch, num_blocks=8):
     pool = GpuKVBlockPool(num_blocks=num_blocks, block_size_tokens=BS, num_layers=1, num_kv_heads=HKV, head_dim=D,
                           dtype=torch.float16, device="cpu")
     pool._ensure_pools()
-    monkeypatch.setattr(pool, "_gathers_on_device", lambda: True)
+    monkeypatch.setattr(pool, "_gathers_on_device", lambda tokens: True)
     return pool
 
 
