@@ -417,8 +417,10 @@ extern "C" int mx_prefill_attn(const uint16_t* q, int64_t q_sb, int64_t q_sh, in
     // A token's row within a head is a 32-bit element offset.
     if ((int64_t)S * k_st > 0x7fffffff || (int64_t)S * v_st > 0x7fffffff)
         return fail(MX_ERR_UNSUPPORTED, "%s: K and V rows of a head must span less than 2^31 elements", what);
-    // Indices of row blocks, units and workgroups stay below 2^31.
-    if ((int64_t)B * Hq * ceil_div((int64_t)P, 16) > (1 << 30) || S > (1 << 30))
+    // A launch holds fewer than 2^32 threads (that many workgroups only with two row tiles per wave,
+    // see launch_qt). Indices of tokens, row blocks, units and workgroups then stay below 2^31.
+    const int64_t wgs = (int64_t)B * Hkv * ceil_div(ceil_div((int64_t)P, 32) * (Hq / Hkv), prefill::kUnits);
+    if (wgs > 0xffffffffll / prefill::kThreads || S > (1 << 30))
         return fail(MX_ERR_UNSUPPORTED, "%s: too many rows", what);
     prefill::Params p{};
     p.q = reinterpret_cast<const _Float16*>(q);

@@ -51,6 +51,13 @@ def _rows_aligned(t: torch.Tensor) -> bool:
             and (n == 1 or sn % 8 == 0))
 
 
+def _prefill_launch_holds(b: int, hkv: int, groups: int, q_len: int, kv_len: int) -> bool:
+    """Whether one launch of ``mx_prefill_attn`` takes these sizes: fewer than 2**32 threads in
+    workgroups of 512 (4 units of 32 query rows of a head each), tokens a 32-bit index."""
+    workgroups = b * hkv * -(-(-(-q_len // 32) * groups) // 4)
+    return workgroups * 512 < 1 << 32 and kv_len <= 1 << 30
+
+
 def _prefill_kernel_takes(query, key, value, scaling, num_kv_groups) -> bool:
     """Whether ``mx_prefill_attn`` gives this call's causal attention. It takes plain device tensors
     outside autograd, tracing, function transforms and autocast (the eager chain is what those
@@ -77,7 +84,7 @@ def _prefill_kernel_takes(query, key, value, scaling, num_kv_groups) -> bool:
             and value.shape == key.shape and key.shape[0] == b and key.shape[3] == d and d in (64, 128)
             and hkv > 0 and hq == hkv * num_kv_groups and b > 0 and 2 <= q_len <= kv_len
             and isinstance(scaling, (int, float)) and 0.0 < scaling < 3e38
-            and b * hq * q_len < 1 << 30 and kv_len < 1 << 30
+            and _prefill_launch_holds(b, hkv, num_kv_groups, q_len, kv_len)
             and kv_len * max(key.stride(2), value.stride(2)) < 1 << 31
             and _rows_aligned(query) and _rows_aligned(key) and _rows_aligned(value))
 

@@ -229,3 +229,26 @@ def test_fused_mlp_rejects_bad_arguments():
     _status(call(kk=1024, ii=4096, nn=1024), _hip.MX_ERR_UNSUPPORTED)  # gate||up would split K there
     assert lib.mx_w8a16_mlp_fused_supported(4, k, i, n) == 0
     assert lib.mx_w8a16_mlp_fused_supported(48, k, i, n) == 0
+
+
+def test_prompt_attention_refuses_what_one_launch_does_not_hold():
+    """Sizes past 2**32 threads are refused before the launch, and the hook does not send them."""
+    from runtime_amd.phase2.block_paged_attention import _prefill_launch_holds
+
+    lib = _hip.load()
+    fake = ctypes.c_void_p(4096)
+
+    def refused(b, hq, hkv, p, s):
+        return lib.mx_prefill_attn(fake, 64, 64, 64, fake, 64, 64, 64, fake, 64, 64, 64, b, hq, hkv, p, s, 64, 0.125, fake,
+                                   fake, 0, None) == _hip.MX_ERR_UNSUPPORTED
+
+    # The first sizes of 2**23 workgroups of 512 threads (4 units of 32 rows of one head's group).
+    for b, hq, hkv, p, s in ((1 << 23, 1, 1, 2, 2), (1 << 20, 8, 8, 32, 32), (1 << 20, 32, 8, 2, 64),
+                             (1, 8, 1, (1 << 27) - 31, 1 << 27), (1, 1, 1, (1 << 30) - 127, 1 << 30)):
+        assert refused(b, hq, hkv, p, s)
+        assert not _prefill_launch_holds(b, hkv, hq // hkv, p, s)
+    assert refused(1, 1, 1, 2, (1 << 30) + 1) and not _prefill_launch_holds(1, 1, 1, 2, (1 << 30) + 1)
+    # The last sizes below.
+    for b, hkv, groups, p, s in (((1 << 23) - 1, 1, 1, 2, 2), (1, 1, 8, (1 << 27) - 64, 1 << 27), (1, 1, 1, 2, 1 << 30),
+                                 ((1 << 23) - 1, 1, 4, 32, 32)):
+        assert _prefill_launch_holds(b, hkv, groups, p, s)
