@@ -267,7 +267,8 @@ int mx_paged_attn_decode_noalloc(const uint16_t* q, int64_t q_sb, int64_t q_sh, 
  * q: fp16 (bf16 with MX_PA_BF16) [B, Hq, P, D] with strides (q_sb, q_sh, q_st, 1);
  * k, v: [B, Hkv, S, D] with their strides; out: [B, P, Hq, D] contiguous;
  * weights: [B, Hq, P, S] contiguous; S >= P, D in {64, 128}, Hq = G * Hkv.
- * Pointers 16-byte aligned, strides non-negative multiples of 8; scale > 0. */
+ * Pointers 16-byte aligned, strides non-negative multiples of 8; scale > 0, a
+ * normal fp32 number also times log2(e). */
 int mx_prefill_attn(const uint16_t* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const uint16_t* k, int64_t k_sb,
                     int64_t k_sh, int64_t k_st, const uint16_t* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int32_t B,
                     int32_t Hq, int32_t Hkv, int32_t P, int32_t S, int32_t D, float scale, uint16_t* out,

@@ -407,7 +407,9 @@ extern "C" int mx_prefill_attn(const uint16_t* q, int64_t q_sb, int64_t q_sh, in
     if (Hkv <= 0 || Hq <= 0 || Hq % Hkv || S < P)
         return fail(MX_ERR_INVALID, "%s: need Hq a multiple of Hkv and S >= P (Hq=%d Hkv=%d P=%d S=%d)", what, Hq, Hkv, P, S);
     if (D != 64 && D != 128) return fail(MX_ERR_UNSUPPORTED, "%s: head_dim %d (64 or 128)", what, D);
-    if (!(scale > 0.0f) || scale > 3.4e38f) return fail(MX_ERR_UNSUPPORTED, "%s: scale must be positive and finite", what);
+    const float scale_log2e = scale * 1.4426950408889634f;
+    if (!(scale >= 1.17549435e-38f) || scale_log2e > 3.4e38f)
+        return fail(MX_ERR_UNSUPPORTED, "%s: scale must be positive and a normal fp32 number, also times log2(e)", what);
     if (flags & ~MX_PA_BF16) return fail(MX_ERR_INVALID, "%s: unknown flags", what);
     const int64_t strides[] = {q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st};
     for (int64_t s : strides)
@@ -439,7 +441,7 @@ extern "C" int mx_prefill_attn(const uint16_t* q, int64_t q_sb, int64_t q_sh, in
     p.G = Hq / Hkv;
     p.P = P;
     p.S = S;
-    p.scale_log2e = scale * 1.4426950408889634f;
+    p.scale_log2e = scale_log2e;
     p.out = reinterpret_cast<_Float16*>(out);
     p.weights = reinterpret_cast<_Float16*>(weights);
     p.heads = B * Hkv;

@@ -63,7 +63,7 @@ def _prefill_kernel_takes(query, key, value, scaling, num_kv_groups) -> bool:
     outside autograd, tracing, function transforms and autocast (the eager chain is what those
     see), of one 16-bit dtype and a supported head_dim, with at least as many keys as queries (a
     query before the first key has no visible token: the eager chain's softmax over nothing) and a
-    positive scale (the kernel masks scaled scores with -inf)."""
+    positive scale (the kernel masks scaled scores with -inf) that fp32 holds, also times log2(e)."""
     for t in (query, key, value):
         if type(t) is not torch.Tensor or not t.is_cuda or t.dim() != 4:
             return False
@@ -83,7 +83,7 @@ def _prefill_kernel_takes(query, key, value, scaling, num_kv_groups) -> bool:
             and query.device == key.device == value.device
             and value.shape == key.shape and key.shape[0] == b and key.shape[3] == d and d in (64, 128)
             and hkv > 0 and hq == hkv * num_kv_groups and b > 0 and 2 <= q_len <= kv_len
-            and isinstance(scaling, (int, float)) and 0.0 < scaling < 3e38
+            and isinstance(scaling, (int, float)) and 2.0**-125 <= scaling <= 2.0**126
             and _prefill_launch_holds(b, hkv, num_kv_groups, q_len, kv_len)
             and kv_len * max(key.stride(2), value.stride(2)) < 1 << 31
             and _rows_aligned(query) and _rows_aligned(key) and _rows_aligned(value))

@@ -252,3 +252,10 @@ def test_prompt_attention_refuses_what_one_launch_does_not_hold():
     for b, hkv, groups, p, s in (((1 << 23) - 1, 1, 1, 2, 2), (1, 1, 8, (1 << 27) - 64, 1 << 27), (1, 1, 1, 2, 1 << 30),
                                  ((1 << 23) - 1, 1, 4, 32, 32)):
         assert _prefill_launch_holds(b, hkv, groups, p, s)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.125, 1e-42, 2.9e38, float("inf"), float("nan")])
+def test_prompt_attention_refuses_scales_fp32_does_not_hold(scale):
+    fake = ctypes.c_void_p(4096)
+    _status(_hip.load().mx_prefill_attn(fake, 64, 64, 64, fake, 64, 64, 64, fake, 64, 64, 64, 1, 1, 1, 2, 2, 64, scale,
+                                        fake, fake, 0, None), _hip.MX_ERR_UNSUPPORTED)

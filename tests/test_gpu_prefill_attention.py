@@ -130,3 +130,23 @@ def test_a_row_whose_visible_scores_are_all_minus_infinity_is_nan_everywhere(dty
     assert weights[0, 1, 0].isnan().all() and out[0, 0, 1].isnan().all()
     assert torch.equal(weights[0, :1], base[1][0]) and torch.equal(out[0, :, :1], base[0][0])
     assert weights[0, 1, 1:].isfinite().all() and out[0, 1:, 1].isfinite().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("scaling", [1e-50, 1e-42, 1e-37, 2.9e38, True])
+def test_any_positive_scale_gives_the_eager_chain_s_weights(dtype, scaling):
+    """Scales that fp32 does not hold, or not times log2(e), are left to the eager chain."""
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(1, 2, 80, 64, generator=g).to(DEV, dtype) for _ in range(3))
+    q, k = q / 64, k / 64
+    if scaling > 1:  # the scores stay finite: 0
+        q = torch.zeros_like(q)
+    out, weights = bpa.block_paged_attention_forward(
+        SimpleNamespace(num_key_value_groups=1, training=False), q, k, v, None, scaling)
+    scores = torch.matmul(q.double().cpu(), k.double().cpu().transpose(2, 3).contiguous()) * scaling
+    w = torch.softmax(scores.masked_fill(bpa._causal_block(80, 80, scores.device), float("-inf")), dim=-1)
+    u, sub = UNIT[dtype]
+    # The eager chain rounds a score twice to the element type: at most 2 u |score| on each exponent.
+    rel = u + 1e-4 + 2 * (2 * u) * scores.abs().max().item()
+    assert ((weights.double().cpu() - w).abs() <= rel * w + sub + 1e-9).all()
+    assert out.isfinite().all()
