@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define MX_ABI_VERSION 19
+#define MX_ABI_VERSION 20
 
 typedef enum mx_status {
     MX_OK = 0,
@@ -64,7 +64,8 @@ int mx_w8a16_quantize(const float* w, int64_t N, int64_t K, int8_t* q, uint16_t*
  * Reference: same load step, worker_server.py:194-205. */
 int mx_w8a16_pack(const int8_t* q, int64_t N, int64_t K, uint8_t* packed, void* stream);
 
-/* Workspace bytes mx_w8a16_linear needs for this shape (0: none). */
+/* Workspace bytes mx_w8a16_linear needs for this shape (0: none). With a smaller
+ * or no workspace it runs in one k range, which sums in another order. */
 size_t mx_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* y[m, n] = fp16( scale[n] * sum_k x[m, k] * q[n, k] + bias[n] ), fp32
@@ -85,6 +86,12 @@ int mx_w8a16_linear(const uint16_t* x, int64_t M, int64_t K, int64_t x_stride, c
  * Returns 1 for M > 128, where no partials entry exists (mx_w8a16_linear runs
  * one launch over all rows, its k ranges within the workspace of 128 rows). */
 int mx_w8a16_splits(int64_t M, int64_t N, int64_t K);
+
+/* How mx_w8a16_linear (gateup = 0) or mx_w8a16_gateup_swiglu (gateup != 0, N = 2 I)
+ * runs M contiguous rows in its one many-row launch: 16-row tiles per workgroup
+ * | n-tiles per wave << 8 | k ranges << 16, or 0 where it takes its other launches.
+ * Host arithmetic only; for tests of the choice. */
+int mx_w8a16_rows_plan(int64_t M, int64_t N, int64_t K, int32_t gateup);
 
 /* The split-K part of mx_w8a16_linear without the reduction:
  * partials[s][m][n] = scale[n] * sum over the k of split s of x[m, k] q[n, k]

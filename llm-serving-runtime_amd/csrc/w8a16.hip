@@ -810,6 +810,13 @@ static size_t workspace_for(int M, int NT, int KT) {
     return pl.KS > 1 ? (size_t)pl.KS * M * NT * kTileN * sizeof(float) : 0;
 }
 
+// The many-row launch's plan of a call, MT = 0 where this file's launches run it. Its k ranges
+// stay within the workspace of a kMaxRows-row call.
+static RowsPlan rows_plan_for(bool gu, int64_t M, int64_t xs, int NT, int KT) {
+    if (M <= (gu ? kGateupMaxRows : kMaxRows) || !rows_fit(M, xs, NT)) return RowsPlan{0, 0, 1};
+    return plan_rows(M, NT, KT, gu ? 0 : workspace_for(kMaxRows, NT, KT));
+}
+
 template <int M, bool GU = false>
 static void launch_gemv(const uint16_t* x, int64_t xs, const uint8_t* w, const uint16_t* s, const uint16_t* b,
                         uint16_t* y, int64_t ys, int NT, int KT, hipStream_t st) {
@@ -1116,6 +1123,14 @@ extern "C" size_t mx_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     return w8a16::workspace_for(mc, (int)(N / w8a16::kTileN), (int)(K / w8a16::kTileK));
 }
 
+extern "C" int mx_w8a16_rows_plan(int64_t M, int64_t N, int64_t K, int32_t gateup) {
+    if (M <= 0 || N <= 0 || K <= 0 || N % w8a16::kTileN || K % w8a16::kTileK) return 0;
+    if (N / w8a16::kTileN > 0x7fffffff || K * 64 > 0x7fffffff) return 0;
+    const w8a16::RowsPlan rp =
+        w8a16::rows_plan_for(gateup != 0, M, K, (int)(N / w8a16::kTileN), (int)(K / w8a16::kTileK));
+    return rp.MT | rp.NPW << 8 | (rp.MT ? rp.KS : 0) << 16;
+}
+
 extern "C" int mx_w8a16_linear(const uint16_t* x, int64_t M, int64_t K, int64_t x_stride, const uint8_t* packed,
                                const uint16_t* scale, const uint16_t* bias, uint16_t* y, int64_t N, int64_t y_stride,
                                void* workspace, size_t workspace_bytes, void* stream) {
@@ -1138,10 +1153,9 @@ extern "C" int mx_w8a16_linear(const uint16_t* x, int64_t M, int64_t K, int64_t 
     const int KT = (int)(K / w8a16::kTileK);
     hipStream_t st = as_stream(stream);
     float* partial = static_cast<float*>(workspace);
-    if (M > w8a16::kMaxRows && w8a16::rows_fit(M, x_stride, NT)) {
-        // Planned from the bytes the call may ask for, not from those it got: the same shape always
-        // takes the same ranges.
-        w8a16::RowsPlan rp = w8a16::plan_rows(M, NT, KT, mx_w8a16_workspace_bytes(M, N, K));
+    w8a16::RowsPlan rp = w8a16::rows_plan_for(false, M, x_stride, NT, KT);
+    if (rp.MT) {
+        // Planned from the bytes the call may ask for; one range where it got fewer.
         if (rp.KS > 1 && (!workspace || workspace_bytes < (size_t)rp.KS * M * N * sizeof(float)))
             rp = w8a16::plan_rows(M, NT, KT, 0);
         w8a16::launch_rows(false, rp, x, x_stride, (int)M, packed, scale, bias, y, y_stride, NT, KT, partial, st);
@@ -1276,9 +1290,9 @@ extern "C" int mx_w8a16_gateup_swiglu(const uint16_t* x, int64_t M, int64_t K, i
     // shapes one launch without K split costs less than a split launch plus a SwiGLU launch
     // (the Qwen2-0.5B MLP at batch 16).
     hipStream_t st = as_stream(stream);
-    if (M > w8a16::kGateupMaxRows && w8a16::rows_fit(M, x_stride, NT)) {
-        w8a16::launch_rows(true, w8a16::plan_rows(M, NT, KT, 0), x, x_stride, (int)M, packed, scale, bias, y, y_stride,
-                           NT, KT, nullptr, st);
+    const w8a16::RowsPlan rp = w8a16::rows_plan_for(true, M, x_stride, NT, KT);
+    if (rp.MT) {
+        w8a16::launch_rows(true, rp, x, x_stride, (int)M, packed, scale, bias, y, y_stride, NT, KT, nullptr, st);
         return check_launch("mx_w8a16_gateup_swiglu");
     }
     for (int64_t m0 = 0; m0 < M; m0 += w8a16::kGateupMaxRows) {

@@ -7,7 +7,7 @@ namespace mx {
 namespace w8a16 {
 
 struct RowsPlan {
-    int MT;   // 16-row tiles per workgroup
+    int MT;   // 16-row tiles per workgroup; 0: the shape is not for this launch
     int NPW;  // n-tiles per wave (4 waves per workgroup)
     int KS;   // k ranges; more than one writes fp32 partials [KS][M][N]
 };

@@ -15,7 +15,7 @@ import threading
 import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "libmxdecode.so")
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 MX_OK = 0
 MX_ERR_INVALID = -1
@@ -41,6 +41,7 @@ SIGNATURES = {
     "mx_w8a16_pack": (ctypes.c_int, [_p, _i64, _i64, _p, _p]),
     "mx_w8a16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "mx_w8a16_linear": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _sz, _p]),
+    "mx_w8a16_rows_plan": (ctypes.c_int, [_i64, _i64, _i64, _i32]),
     "mx_w8a16_splits": (ctypes.c_int, [_i64, _i64, _i64]),
     "mx_w8a16_linear_partials": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _p, _i64, _p, _sz, _p]),
     "mx_w8a16_linear_swiglu": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _sz, _p]),

@@ -35,16 +35,29 @@ def _product(x, w, bias=None):
     return y, U * y.abs() + SUB + (x.shape[1] + 2) * 2.0**-24 * mag
 
 
-# Every row tile (32, 64, 96, 128 rows) and both widths (128 and 256 channels) with remainders, n-tiles
-# past the last one, one k-tile, k-tile counts around the unrolled loops' 2, 3 and 12, and shapes that
-# split K.
-@pytest.mark.parametrize("m,n,k,bias", [
+# Every instance of the launch (row tiles of 32, 64, 96 and 128 rows, 128 and 256 channels) with remainders
+# of both, n-tiles past the last one, one k-tile, k-tile counts around the unrolled loops' 2, 3 and 12, and
+# shapes that split K; test_int8_rows_plan.py checks that these shapes still reach them.
+LINEAR = [
     (129, 1152, 896, True), (777, 1152, 896, True), (160, 4096, 4096, False), (256, 896, 4864, True),
     (1531, 4096, 1024, False), (2049, 4112, 192, True), (1000, 16, 64, False), (130, 272, 64, True),
     (385, 6144, 4096, False), (4096, 2048, 128, False), (191, 4096, 14336, False),
     (256, 4096, 14336, False), (1531, 4096, 14336, False), (700, 28672, 832, True), (2048, 28672, 1600, False),
     (130, 6144, 704, False), (140, 2048, 768, True), (150, 1024, 1600, False),
-])
+    (4167, 832, 832, True), (300, 4096, 4096, False), (198, 28560, 960, False), (4218, 784, 1792, False),
+    (2814, 17568, 1920, False), (2814, 17568, 1984, True), (164, 22208, 1792, False),
+    (3377, 528, 1856, True),
+]
+GATEUP = [
+    (65, 4864, 896, False), (128, 4864, 896, True), (129, 4864, 896, False), (777, 1032, 192, True),
+    (2048, 14336, 256, False), (300, 14336, 4096, False), (150, 8, 64, False), (96, 14336, 4096, False),
+    (128, 14336, 4096, True), (66, 5632, 2048, False), (2000, 14336, 1088, False), (64, 4864, 896, False),
+    (98, 12560, 128, False), (260, 14336, 4096, True), (4167, 416, 832, True), (198, 14280, 960, False),
+    (71, 10912, 1920, False), (4218, 392, 1792, False), (2814, 8784, 1920, True), (2814, 8784, 1984, False), (164, 11104, 1792, True),
+]
+
+
+@pytest.mark.parametrize("m,n,k,bias", LINEAR)
 def test_linear(m, n, k, bias):
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     q, scale, w = _weights(n, k, g)
@@ -78,11 +91,7 @@ def test_without_workspace_runs_in_one_range():
     assert ((y.double() - want).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("m,inter,k,bias", [
-    (65, 4864, 896, False), (128, 4864, 896, True), (129, 4864, 896, False), (777, 1032, 192, True),
-    (2048, 14336, 256, False), (300, 14336, 4096, False), (150, 8, 64, False), (96, 14336, 4096, False),
-    (128, 14336, 4096, True), (66, 5632, 2048, False), (2000, 14336, 1088, False), (64, 4864, 896, False),
-])
+@pytest.mark.parametrize("m,inter,k,bias", GATEUP)
 def test_gateup(m, inter, k, bias):
     g = torch.Generator(device=DEV).manual_seed(m + inter + k)
     parts = [_weights(inter, k, g) for _ in range(2)]
