@@ -275,7 +275,9 @@ int mx_paged_attn_decode_noalloc(const uint16_t* q, int64_t q_sb, int64_t q_sh, 
  * k, v: [B, Hkv, S, D] with their strides; out: [B, P, Hq, D] contiguous;
  * weights: [B, Hq, P, S] contiguous; S >= P, D in {64, 128}, Hq = G * Hkv.
  * Pointers 16-byte aligned, strides non-negative multiples of 8; scale > 0, a
- * normal fp32 number also times log2(e). */
+ * normal fp32 number also times log2(e). Where v[j] is not finite, the eager
+ * chain's 0 * v[j] is NaN for every row that does not see j; here for those rows
+ * only whose own last 64-token tile holds j. */
 int mx_prefill_attn(const uint16_t* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const uint16_t* k, int64_t k_sb,
                     int64_t k_sh, int64_t k_st, const uint16_t* v, int64_t v_sb, int64_t v_sh, int64_t v_st, int32_t B,
                     int32_t Hq, int32_t Hkv, int32_t P, int32_t S, int32_t D, float scale, uint16_t* out,

@@ -5,20 +5,23 @@
 // A workgroup of 4 waves computes MT * 16 rows x 256 or 128 channels. Each wave owns NPW = 4 or 2
 // n-tiles for all of the workgroup's rows, so a weight byte is loaded and dequantized once per
 // workgroup, straight into the registers that the MFMAs read. x goes through LDS, its 16-byte chunks
-// swapped round by the row's low bits so that neither the stores nor the fragment reads meet in a
-// bank; every fragment feeds NPW n-tiles. The products are taken transposed (weights as the A operand),
-// so that a lane ends up with 4 consecutive channels of one row and stores 8 bytes (16 of a split's
-// partial). Stages are selected by compile-time indices in an unrolled loop: a copy between stages made
-// the compiler wait for the loads where they were issued.
+// swapped round by the row's low three bits: the stores meet in no bank, a fragment read meets twice
+// (rows r and r + 8; the counters call 4 of its 8 LDS cycles conflicts). Every fragment feeds NPW
+// n-tiles. The products are taken transposed (weights as the A operand), so that a lane ends up with 4
+// consecutive channels of one row and stores 8 bytes (16 of a split's partial). Stages are selected by
+// compile-time indices in an unrolled loop: a copy between stages made the compiler wait for the loads
+// where they were issued.
 //
 // Few workgroups per CU are bound by their own chain (barrier, x store, fragment reads, dequant,
 // products), so each half k-tile's fragments and weights are made ready under the previous half's
 // products: 0.47-0.60 -> 0.43-0.53 us per k-tile for one workgroup of 32 or 64 rows x 256 channels, and
 // 0.25-0.34 us with 128 channels. Many are bound by the matrix cores together with what feeds them.
-// Llama-3-8B gate||up at 2048 rows: 646-668 -> 416-431 us (720-744 -> 1115-1155 TFLOP/s; torch's fp16
-// product of that size takes 418 us). The MFMAs and barriers alone take 272 us; without the dequant it would be 385, without
-// the weight loads 323-360, without the x loads 374. Loads two or three k-tiles ahead measured the
-// same, 8 waves per workgroup (128 x 512 or 256 x 256) 440-500 us: one barrier then holds the whole CU.
+// Llama-3-8B gate||up at 2048 rows: 646-680 -> 416-445 us (707-744 -> 1081-1155 TFLOP/s; torch's fp16
+// product of that size takes 418 us). The MFMAs and barriers alone take 272 us; without the dequant it
+// would be 385, without the weight loads 323-360, without the x loads 374. Counters there: MFMA busy
+// 59 %, 4.55 GB read out of L2 per call (10.4 TB/s), 71 % of the requests hits. Loads two or three
+// k-tiles ahead measured the same, 8 waves per workgroup (128 x 512 or 256 x 256) 440-500 us: one barrier
+// then holds the whole CU.
 #include "w8a16_rows.h"
 
 #include "w8a16_tiles.h"
@@ -189,7 +192,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemm_rows_kernel(
         // 8 x 4 tiles per wave hold 128 accumulators: no registers for that. Step j stores x k-tile
         // j + 1 (loaded a step ago) into the other buffer, whose readers passed the last barrier,
         // issues the loads of the next stages and computes k-tile j, ahead of the other workgroup's
-        // waves on the SIMD while they do the rest (418 against 426 us at 2048 rows).
+        // waves on the SIMD while they do the rest (4096 x 14336 at 4096 rows 413-415 against 421 us
+        // without the priority; 6144 x 4096 there and gate||up 28672 x 4096 at 1100 rows the same).
         store_x(0, load_x(0));
         WStage w0 = load_w(0), w1;
         XStage xn = load_x(1);
